@@ -396,7 +396,8 @@ hipError_t launch_accumulate(const DevSensor& S, const float* x, const float* y,
 // LEAN: the launch accumulates into one LDS image per block with wave-merged
 // adds (the batched forward and the default sample-major image); the other
 // accumulation paths are compiled out, which keeps scalar registers free.
-template <int SRC, int KIND, int SPLAT, int MODE, bool STAGES, bool AXIS, bool LEAN = false>
+// OBST: as in primary_shadow (an image without obstructions has no shadow code).
+template <int SRC, int KIND, int SPLAT, int MODE, bool STAGES, int OBST, bool LEAN = false>
 __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace(TraceArgs A) {
   extern __shared__ float smem[];
   const bool lds_image = LEAN || A.lds_image;
@@ -474,7 +475,7 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace(TraceArgs A) {
       // prefetch the next value while this source is traced
       const float nv = vals[s + 1 < s1 ? s + 1 : s];
       float gu, gv, v, x, y;
-      const bool ok = trace_ray<SRC, KIND, STAGES, AXIS, 2, MODE == IACT_MODE_DEBUG>(
+      const bool ok = trace_ray<SRC, KIND, STAGES, false, OBST, MODE == IACT_MODE_DEBUG>(
           A, smp, active, e, source_qs(A, e), sv, gu, gv, v, x, y);
       sv = nv;
       if (MODE == IACT_MODE_DEBUG) {
@@ -1340,17 +1341,18 @@ hipError_t launch_world(const iact_facets& F, const DevSensor& S, float* out, hi
 // through pick_trace_kernel, so the grid is sized for the kernel that runs.
 template <int SRC, int KIND, int SPLAT, int MODE>
 static TraceKernel pick_trace_t(const TraceArgs& A) {
-  // image mode is specialised for primary-only scenes and identity sensor
-  // frames; both specialisations compute bit-identical results to the
+  // image mode is specialised for primary-only scenes, with and without
+  // obstructions; the specialisations compute bit-identical results to the
   // generic kernel, they only skip instructions
   if (MODE == IACT_MODE_IMAGE && A.n_stages == 0) {
+    const bool ob = has_obstructions(A.ob);
     if (A.lds_image && A.acc == 0 && !A.det)
-      return A.S.axis ? k_trace<SRC, KIND, SPLAT, MODE, false, true, true>
-                      : k_trace<SRC, KIND, SPLAT, MODE, false, false, true>;
-    return A.S.axis ? k_trace<SRC, KIND, SPLAT, MODE, false, true>
-                    : k_trace<SRC, KIND, SPLAT, MODE, false, false>;
+      return ob ? k_trace<SRC, KIND, SPLAT, MODE, false, 1, true>
+                : k_trace<SRC, KIND, SPLAT, MODE, false, 0, true>;
+    return ob ? k_trace<SRC, KIND, SPLAT, MODE, false, 1>
+              : k_trace<SRC, KIND, SPLAT, MODE, false, 0>;
   }
-  return k_trace<SRC, KIND, SPLAT, MODE, true, false>;
+  return k_trace<SRC, KIND, SPLAT, MODE, true, 2>;
 }
 
 // source-major kernels exist for primary-only scenes (the host selects that

@@ -508,8 +508,18 @@ CullLayout cull_layout(int nf, int words, int all, size_t base, const CullSpec& 
 // culling tables (256-B aligned): n_images * n_pixels doubles.
 size_t image64_offset(size_t end) { return align256(end); }
 
-size_t workspace_bytes_for(const iact_scene& sc, int ns, int mode, const LaunchShape& shp,
-                           const TraceArgs& A) {
+// Workspace of an image render through the spot tree: its layout, then the
+// fp64 sums.
+static size_t tree_workspace_bytes(const iact_scene& sc, const TreeLayout& T) {
+  return T.sums + (size_t)sc.sensor.n_pixels * sizeof(double);
+}
+
+// tree: the render takes the spot tree where that serves it
+static size_t workspace_bytes_for(const iact_scene& sc, int ns, int mode, const LaunchShape& shp,
+                                  const TraceArgs& A, const DevInfo& dev, bool tree) {
+  LaunchShape ts;
+  if (mode == IACT_MODE_IMAGE && tree && tree_serves(A, 0, dev, ts))
+    return tree_workspace_bytes(sc, tree_layout(sc, ns, tree_sorts(A, ns)));
   const size_t base = base_workspace_bytes(sc, mode, shp, A);
   const CullSpec c{ns, 1, nullptr, mode == IACT_MODE_IMAGE && !A.det, refine_groups(A, mode)};
   const size_t end = cull_layout(A.nf, A.cull_words, A.cull_all, base, c).end;
@@ -583,6 +593,12 @@ int adj_sm_layout(const iact_scene& sc, const double* sources, const float* valu
   const size_t end = cull_layout(A.nf, A.cull_words, A.cull_all, out.recs_end, c).end;
   out.torque = align256(end);
   out.end = out.torque + (size_t)3 * sc.facets.n_facets * sizeof(double);
+  LaunchShape ts;
+  if (tree_serves(A, 1, dev, ts)) {
+    const size_t t = tree_layout(sc, ns, tree_sorts(A, ns)).sums +
+                     (size_t)3 * sc.facets.n_facets * sizeof(double);
+    if (t > out.end) out.end = t;
+  }
   return IACT_OK;
 }
 
@@ -696,8 +712,8 @@ int32_t iact_facet_world(const iact_facets* F, float* out, void* stream) {
   return e == hipSuccess ? IACT_OK : hip_error(e, "k_facet_world");
 }
 
-size_t iact_workspace_size(const iact_scene* scene, int32_t n_sources, int32_t mode,
-                           const iact_launch* launch) {
+static size_t workspace_size(const iact_scene* scene, int32_t n_sources, int32_t mode,
+                             const iact_launch* launch, bool tree) {
   if (validate_scene(scene) || n_sources < 0) return 0;
   DevInfo dev;
   if (device_info(dev)) return 0;
@@ -705,13 +721,19 @@ size_t iact_workspace_size(const iact_scene* scene, int32_t n_sources, int32_t m
   fill_trace_args(A, *scene, nullptr, nullptr, n_sources);
   LaunchShape shp;
   if (shape_trace(*scene, n_sources, mode, launch, A, shp, dev, -1)) return 0;
-  return workspace_bytes_for(*scene, n_sources, mode, shp, A);
+  return workspace_bytes_for(*scene, n_sources, mode, shp, A, dev, tree);
 }
 
-int32_t iact_trace_fwd(const iact_scene* scene, const double* sources, const float* values,
-                       int32_t n_sources, int32_t source_type, int32_t mode,
-                       const iact_launch* launch, void* workspace, size_t workspace_bytes,
-                       float* out, float* debug_xy, int32_t* debug_pixel, void* stream) {
+size_t iact_workspace_size(const iact_scene* scene, int32_t n_sources, int32_t mode,
+                           const iact_launch* launch) {
+  return workspace_size(scene, n_sources, mode, launch, true);
+}
+
+static int32_t trace_fwd(const iact_scene* scene, const double* sources, const float* values,
+                         int32_t n_sources, int32_t source_type, int32_t mode,
+                         const iact_launch* launch, void* workspace, size_t workspace_bytes,
+                         float* out, float* debug_xy, int32_t* debug_pixel, void* stream,
+                         bool want_tree) {
   int rc = validate_scene(scene);
   if (rc) return rc;
   if (n_sources < 0) return set_error(IACT_ERR_INVALID, "negative source count");
@@ -738,7 +760,7 @@ int32_t iact_trace_fwd(const iact_scene* scene, const double* sources, const flo
   LaunchShape shp;
   rc = shape_trace(sc, n_sources, mode, launch, A, shp, dev, source_type);
   if (rc) return rc;
-  const size_t need = workspace_bytes_for(sc, n_sources, mode, shp, A);
+  const size_t need = workspace_bytes_for(sc, n_sources, mode, shp, A, dev, want_tree);
   if (need > 0 && (!workspace || workspace_bytes < need))
     return set_error(IACT_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need,
                      workspace_bytes);
@@ -747,6 +769,20 @@ int32_t iact_trace_fwd(const iact_scene* scene, const double* sources, const flo
   A.dbg_pix = debug_pixel;
   hipError_t e = hipSuccess;
   const bool empty = (sc.facets.n_facets == 0 || n_sources == 0);
+  LaunchShape tshp;
+  if (mode == IACT_MODE_IMAGE && !empty && want_tree && tree_serves(A, 0, dev, tshp)) {
+    const TreeLayout T = tree_layout(sc, n_sources, tree_sorts(A, n_sources));
+    AdjArgs B;
+    memset(&B, 0, sizeof(B));
+    B.T = A;
+    B.T.out64 = (double*)((char*)workspace + T.sums);
+    e = launch_fill_d(B.T.out64, P, 0.0, st);
+    if (e != hipSuccess) return hip_error(e, "clear image sums");
+    rc = launch_tree(B, T, workspace, tshp, source_type, 0, st);
+    if (rc) return rc;
+    e = launch_f64_to_f32(B.T.out64, out, P, st);
+    return e == hipSuccess ? IACT_OK : hip_error(e, "k_f64_to_f32");
+  }
   if (!empty) {
     const CullSpec c{n_sources, 1, nullptr, mode == IACT_MODE_IMAGE && !A.det,
                      refine_groups(A, mode)};
@@ -812,6 +848,14 @@ int32_t iact_trace_fwd(const iact_scene* scene, const double* sources, const flo
   return e == hipSuccess ? IACT_OK : hip_error(e, "k_trace(debug)");
 }
 
+int32_t iact_trace_fwd(const iact_scene* scene, const double* sources, const float* values,
+                       int32_t n_sources, int32_t source_type, int32_t mode,
+                       const iact_launch* launch, void* workspace, size_t workspace_bytes,
+                       float* out, float* debug_xy, int32_t* debug_pixel, void* stream) {
+  return trace_fwd(scene, sources, values, n_sources, source_type, mode, launch, workspace,
+                   workspace_bytes, out, debug_xy, debug_pixel, stream, true);
+}
+
 // ------------------------------------------------------- no-allocation entry
 // Scratch of iact_trace_fwd_noalloc: a file-scope device array, one copy per
 // GPU (each device's code object holds its own), kept until the process
@@ -856,8 +900,14 @@ int32_t iact_trace_fwd_noalloc(const iact_scene* scene, const double* sources,
   // needs more than the scratch holds (the source-major record table, 64 B
   // per sample) takes the sample-major layout, which has none
   iact_launch L = launch ? *launch : iact_launch{};
-  // (a size of 0 from an invalid launch: iact_trace_fwd reports the error)
-  size_t need = iact_workspace_size(scene, n_sources, mode, &L);
+  // (a size of 0 from an invalid launch: iact_trace_fwd reports the error);
+  // between the two lies the source-major trace without the spot tree's nodes
+  bool tree = true;
+  size_t need = workspace_size(scene, n_sources, mode, &L, true);
+  if (need > (size_t)IACT_NOALLOC_SCRATCH_BYTES && mode == IACT_MODE_IMAGE) {
+    tree = false;
+    need = workspace_size(scene, n_sources, mode, &L, false);
+  }
   if (need > (size_t)IACT_NOALLOC_SCRATCH_BYTES && mode == IACT_MODE_IMAGE && L.layout == 0) {
     L.layout = 1;
     need = iact_workspace_size(scene, n_sources, mode, &L);
@@ -870,8 +920,8 @@ int32_t iact_trace_fwd_noalloc(const iact_scene* scene, const double* sources,
   void* ws = nullptr;
   rc = scratch_address(&ws);
   if (rc) return rc;
-  return iact_trace_fwd(scene, sources, values, n_sources, source_type, mode, &L, ws,
-                        (size_t)IACT_NOALLOC_SCRATCH_BYTES, out, debug_xy, debug_pixel, stream);
+  return trace_fwd(scene, sources, values, n_sources, source_type, mode, &L, ws,
+                   (size_t)IACT_NOALLOC_SCRATCH_BYTES, out, debug_xy, debug_pixel, stream, tree);
 }
 
 }  // extern "C"

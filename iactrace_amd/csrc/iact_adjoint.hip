@@ -672,6 +672,25 @@ int32_t iact_trace_bwd(const iact_scene* scene, const double* sources, const flo
     if (lay.end > 0 && (!workspace || workspace_bytes < lay.end))
       return set_error(IACT_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", lay.end,
                        workspace_bytes);
+    B.grad_image = grad_image;
+    B.g_pos = grads->positions;
+    B.g_src = grads->sources;
+    B.g_val = grads->values;
+    const int mode = B.g_pos || B.g_src || B.g_val ? 2 : 1;
+    LaunchShape tshp;
+    if (tree_serves(A, mode, dev, tshp)) {
+      const TreeLayout T = tree_layout(sc, n_sources, tree_sorts(A, n_sources));
+      B.torque = (double*)((char*)workspace + T.sums);
+      e = launch_fill_d(B.torque, 3ll * nf, 0.0, st);
+      if (e != hipSuccess) return hip_error(e, "clear torques");
+      rc = launch_tree(B, T, workspace, tshp, source_type, mode, st);
+      if (rc) return rc;
+      if (grads->rotations) {
+        e = launch_torque_to_euler(B.torque, sc.facets.rotations, nf, grads->rotations, st);
+        if (e != hipSuccess) return hip_error(e, "k_torque_to_euler");
+      }
+      return IACT_OK;
+    }
     const size_t tab = hex_table_bytes(sc.sensor);
     shp.lds = (size_t)(sc.sensor.n_pixels + 1) * sizeof(float) + tab;  // G[-1] = 0 + G
     if (shp.lds > 65536)
@@ -690,10 +709,6 @@ int32_t iact_trace_bwd(const iact_scene* scene, const double* sources, const flo
     B.torque = (double*)((char*)workspace + lay.torque);
     e = launch_fill_d(B.torque, 3ll * nf, 0.0, st);
     if (e != hipSuccess) return hip_error(e, "clear torques");
-    B.grad_image = grad_image;
-    B.g_pos = grads->positions;
-    B.g_src = grads->sources;
-    B.g_val = grads->values;
     e = launch_adjoint_sm(B, shp, source_type, st);
     if (e != hipSuccess) return hip_error(e, "k_adj_sm");
     if (grads->rotations) {

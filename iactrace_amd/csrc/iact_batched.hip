@@ -179,7 +179,11 @@ static size_t instance_need(const iact_scene* scene, long long ns, int words, in
   const long long total = (long long)scene->facets.n_facets * scene->facets.n_samples;
   const CullSpec c{ns, 1, nullptr, true, (total + 63) / 64};
   const size_t end = cull_layout(scene->facets.n_facets, words, all, recs, c).end;
-  return image64_offset(end) + (size_t)scene->sensor.n_pixels * sizeof(double);
+  const size_t old = image64_offset(end) + (size_t)scene->sensor.n_pixels * sizeof(double);
+  // (the spot tree sorts from kChunkCullMinSources sources of obstructed scenes)
+  const size_t tree = tree_layout(*scene, (int)ns, words > 0).sums +
+                      (size_t)scene->sensor.n_pixels * sizeof(double);
+  return tree > old ? tree : old;
 }
 
 // Workspace end of the batched kernels' tables (prefix, instance table,

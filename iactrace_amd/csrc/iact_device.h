@@ -298,14 +298,25 @@ IACT_DEV bool cyl_far(f3 oc, const CylDir& D, float r) {
   const float ow = dot(oc, D.w);
   return ow * ow > D.ww * fmaf(1e-5f, dot(oc, oc), 1.0002f * r * r);
 }
+// Axial split of an origin oc relative to the cylinder's first end.
+IACT_DEV void cyl_axial(f3 oc, f3 ax, float r, float& oca, f3& ocp, float& cc) {
+  oca = dot(oc, ax);
+  ocp = oc - oca * ax;
+  cc = dot(ocp, ocp) - r * r;
+}
+// Discriminant of the side hit and its linear term.
+IACT_DEV float cyl_disc(f3 ocp, float cc, const CylDir& D, float& b) {
+  b = 2.f * dot(ocp, D.rdp);
+  return b * b - 4.f * D.a * cc;
+}
 // The side and cap hits from the origin's axial split (oca = oc.ax,
 // ocp = oc - oca ax, cc = |ocp|^2 - r^2) and the direction terms.
 IACT_DEV float cyl_rest(f3 ocp, float oca, float cc, const CylDir& D, float h, float r,
                         bool far) {
   const float eps = 1e-8f;
   const float inf = __builtin_inff();
-  const float b = 2.f * dot(ocp, D.rdp);
-  const float disc = b * b - 4.f * D.a * cc;
+  float b;
+  const float disc = cyl_disc(ocp, cc, D, b);
   const float sq = fsqrt(fmaxf(disc, 0.f));
   float t1 = (-b - sq) * D.ia, t2 = (-b + sq) * D.ia;
   const float y1 = oca + t1 * D.rda, y2 = oca + t2 * D.rda;
@@ -324,9 +335,9 @@ IACT_DEV float hit_cylinder_dir(f3 o, const CylDir& D, cptr<float> c) {
   const f3 oc = o - p1;
   const bool far = cyl_far(oc, D, r);
   if (__all(far)) return __builtin_inff();
-  const float oca = dot(oc, ax);
-  const f3 ocp = oc - oca * ax;
-  const float cc = dot(ocp, ocp) - r * r;
+  float oca, cc;
+  f3 ocp;
+  cyl_axial(oc, ax, r, oca, ocp, cc);
   return cyl_rest(ocp, oca, cc, D, h, r, far);
 }
 // hit_cylinder_dir for two directions from one origin: the origin's terms
@@ -340,9 +351,9 @@ IACT_DEV void hit_cylinder_dir2(f3 o, const CylDir& D0, const CylDir& D1, cptr<f
   const bool far0 = cyl_far(oc, D0, r), far1 = cyl_far(oc, D1, r);
   t0 = t1 = __builtin_inff();
   if (__all(far0 && far1)) return;
-  const float oca = dot(oc, ax);
-  const f3 ocp = oc - oca * ax;
-  const float cc = dot(ocp, ocp) - r * r;
+  float oca, cc;
+  f3 ocp;
+  cyl_axial(oc, ax, r, oca, ocp, cc);
   if (!__all(far0)) t0 = cyl_rest(ocp, oca, cc, D0, h, r, far0);
   if (!__all(far1)) t1 = cyl_rest(ocp, oca, cc, D1, h, r, far1);
 }

@@ -8,6 +8,8 @@
 // wave are merged before touching the LDS image.
 #pragma once
 
+#include <type_traits>
+
 #include "iact_device.h"
 
 namespace iact {
@@ -46,6 +48,25 @@ struct InstDesc {
 };
 static_assert(sizeof(InstDesc) == 32 && offsetof(InstDesc, sbase) == 24,
               "decode_item reads InstDesc as 8 words");
+
+// The spot tree of a primary-only, hard-binned image trace (iact_tree.hip).
+// A node is a run of consecutive sample records of one facet: 1024 (top), 64
+// (patch) or 16 (leaf); a facet's nodes are stored tops, patches, leaves.
+#define IACT_NODE_WORDS 32
+constexpr int kTopSamples = 1024, kPatchSamples = 64, kLeafSamples = 16;
+constexpr int kTreeSources = 512;  // sources of a work item, and threads of a block
+struct TreeParams {
+  const float* nodes;    // (nf * per_facet, IACT_NODE_WORDS)
+  const float* balls;    // (nf * per_facet, 4) bounding balls of the nodes' points
+  const float* frame;    // reference direction (see k_tree_frame)
+  const int16_t* table;  // staged hexagonal table (see k_tree_frame)
+  int n_top, n_patch, n_leaf, per_facet;  // nodes per facet
+  uint32_t n_sb, items;                   // source blocks, work items
+  FastDiv d_sb, d_top;                    // divide by n_sb, by n_top
+  float b0[3], b1[3], b2[3];  // columns of the inverse of the rows (An, Au, Av)
+  float n_au, n_av;           // |Au|, |Av|
+  float hu, hv;               // half a pixel less the edge, in the test's forms
+};
 
 struct TraceArgs {
   // stage-0 facets (local frame samples + pose)
@@ -560,13 +581,21 @@ IACT_DEV float primary_shadow(const TraceArgs& A, const Sample& s, f3 d, bool ac
 // within R of b?  Along the axis the ray point lies in [-rho + t cos, rho + t],
 // across it within rho + t sin of the axis, so it is necessary that
 // s + rho + R >= 0 and e <= rho + R + tan(theta) (s + rho + R), with s, e the
-// axial and radial coordinates of b.  Radii get 0.1% + 1 mm of slack.
+// axial and radial coordinates of b.  Radii get 0.1% + 1 mm of slack, and
+// that of the ray tests' own rounding: a discriminant formed from terms of
+// size |oc|^2 (oc from the obstruction to the ray's origin) moves the squared
+// distance of closest approach by up to some 13 2^-24 |oc|^2, so a thin member
+// far away may be hit by rays that pass centimetres off it.
+IACT_DEV float reach_radius(float r, f3 w, float rho) {
+  const float oc = sqrtf(dot(w, w)) + rho;
+  return fmaf(sqrtf(fmaf(1.5e-6f * oc, oc, r * r)), 1.001f, 1e-3f);
+}
 IACT_DEV bool bundle_reaches(f3 c, float rho, f3 a, float tn, f3 b, float R) {
   const f3 w = b - c;
   const float s = dot(w, a);
   const f3 perp = fma3(-s, a, w);
   const float e = sqrtf(dot(perp, perp));
-  const float rr = fmaf(R, 1.001f, 1e-3f) + rho;
+  const float rr = reach_radius(R, w, rho) + rho;
   // written so that NaN geometry keeps the candidate
   return !(s + rr < 0.f) && !(e > fmaf(tn, s + rr, rr));
 }
@@ -575,28 +604,32 @@ IACT_DEV bool bundle_reaches(f3 c, float rho, f3 a, float tn, f3 b, float R) {
 // boxes, spheres, oriented boxes, triangles)?  Cylinders are tested as the
 // capsule of their axis segment (cylinder_reaches), the other kinds through
 // a bounding sphere.
-IACT_DEV bool cylinder_reaches(const float* q, f3 c, float rho, f3 a, float tn);
+template <typename Ptr>
+IACT_DEV bool cylinder_reaches(Ptr q, f3 c, float rho, f3 a, float tn);
+// UNI: j is wave-uniform (the rows are read with scalar loads).
+template <bool UNI = false>
 IACT_DEV bool obstruction_reaches(const iact_obstructions& ob, int j, f3 c, float rho, f3 a,
                                   float tn) {
+  using Row = std::conditional_t<UNI, cptr<float>, const float*>;
   const int c0 = ob.n_cylinders, c1 = c0 + ob.n_boxes, c2 = c1 + ob.n_spheres;
   const int c3 = c2 + ob.n_oriented_boxes;
-  if (j < c0) return cylinder_reaches(ob.cylinders + 8 * j, c, rho, a, tn);
+  if (j < c0) return cylinder_reaches((Row)(ob.cylinders + 8 * j), c, rho, a, tn);
   if (j < c1) {
-    const float* q = ob.boxes + 6 * (j - c0);
+    const Row q = (Row)(ob.boxes + 6 * (j - c0));
     const f3 lo = mk3(q[0], q[1], q[2]), hi = mk3(q[3], q[4], q[5]);
     const f3 dd = hi - lo;
     return bundle_reaches(c, rho, a, tn, 0.5f * (lo + hi), 0.5f * sqrtf(dot(dd, dd)));
   }
   if (j < c2) {
-    const float* q = ob.spheres + 4 * (j - c1);
+    const Row q = (Row)(ob.spheres + 4 * (j - c1));
     return bundle_reaches(c, rho, a, tn, mk3(q[0], q[1], q[2]), q[3]);
   }
   if (j < c3) {
-    const float* q = ob.oriented_boxes + 15 * (j - c2);
+    const Row q = (Row)(ob.oriented_boxes + 15 * (j - c2));
     const f3 he = mk3(q[3], q[4], q[5]);
     return bundle_reaches(c, rho, a, tn, mk3(q[0], q[1], q[2]), sqrtf(dot(he, he)));
   }
-  const float* q = ob.triangles + 9 * (j - c3);
+  const Row q = (Row)(ob.triangles + 9 * (j - c3));
   const f3 v0 = mk3(q[0], q[1], q[2]), v1 = mk3(q[3], q[4], q[5]);
   const f3 v2 = mk3(q[6], q[7], q[8]);
   const f3 ctr = (1.f / 3.f) * (v0 + v1 + v2);
@@ -614,11 +647,12 @@ IACT_DEV bool obstruction_reaches(const iact_obstructions& ob, int j, f3 c, floa
 // Q(t) = e(t)^2 - g(t)^2 <= 0 somewhere on the interval where s(t) >= -rr
 // and g(t) >= 0 (ends and the vertex of Q).  Q gets a tolerance of 1e-5 of
 // its terms' magnitude; NaN geometry keeps the candidate.
-IACT_DEV bool cylinder_reaches(const float* q, f3 c, float rho, f3 a, float tn) {
+template <typename Ptr>
+IACT_DEV bool cylinder_reaches(Ptr q, f3 c, float rho, f3 a, float tn) {
   const f3 p1 = mk3(q[0], q[1], q[2]), ax = mk3(q[3], q[4], q[5]);
   const float h = q[6], r = q[7];
-  const float rr = fmaf(r, 1.001f, 1e-3f) + rho;
   const f3 w0 = p1 - c;
+  const float rr = reach_radius(r, w0, rho) + rho;
   const float s0 = dot(w0, a), s1 = dot(ax, a);
   const f3 P0 = fma3(-s0, a, w0), P1 = fma3(-s1, a, ax);
   const float G0 = fmaf(tn, s0 + rr, rr), G1 = tn * s1;
@@ -642,6 +676,28 @@ IACT_DEV bool cylinder_reaches(const float* q, f3 c, float rho, f3 a, float tn) 
       1e-5f * (dot(P0, P0) + G0 * G0 + hh * hh * (dot(P1, P1) + G1 * G1) + 1e-6f);
   if (!(lo <= hi)) return lo != lo || hi != hi;  // empty interval (NaN: keep)
   return !(m > tol);
+}
+
+// obstruction_reaches for parallel rays (a bundle of zero angle) and a
+// wave-uniform j.  A box is tested as itself, grown by the ball's radius (a
+// ray of the ball that meets the box passes within that radius of the ball's
+// central ray), which is much tighter than its bounding sphere.
+IACT_DEV bool line_reaches(const iact_obstructions& ob, int j, f3 c, float rho, f3 a) {
+  const int c0 = ob.n_cylinders, c1 = c0 + ob.n_boxes;
+  if (j < c0) return cylinder_reaches(as_const(ob.cylinders) + 8 * j, c, rho, a, 0.f);
+  if (j >= c1) return obstruction_reaches<true>(ob, j, c, rho, a, 0.f);
+  const cptr<float> q = as_const(ob.boxes) + 6 * (j - c0);
+  const float g = fmaf(rho, 1.001f, 1e-3f + 1e-5f * (fabsf(c.x) + fabsf(c.y) + fabsf(c.z)));
+  // (a direction component of 0 as 1e-9: no 0 * inf)
+  const float ix = frcp(fabsf(a.x) < 1e-9f ? 1e-9f : a.x);
+  const float iy = frcp(fabsf(a.y) < 1e-9f ? 1e-9f : a.y);
+  const float iz = frcp(fabsf(a.z) < 1e-9f ? 1e-9f : a.z);
+  const float x1 = (q[0] - g - c.x) * ix, x2 = (q[3] + g - c.x) * ix;
+  const float y1 = (q[1] - g - c.y) * iy, y2 = (q[4] + g - c.y) * iy;
+  const float z1 = (q[2] - g - c.z) * iz, z2 = (q[5] + g - c.z) * iz;
+  const float tmin = fmaxf(fmaxf(fminf(x1, x2), fminf(y1, y2)), fminf(z1, z2));
+  const float tmax = fminf(fminf(fmaxf(x1, x2), fmaxf(y1, y2)), fmaxf(z1, z2));
+  return !(tmax < tmin) && !(tmax < -g);  // (NaN geometry keeps the candidate)
 }
 
 // Shadow bits of a facet run of far sources (source_qs 0): bit i is set when

@@ -508,18 +508,12 @@ CullLayout cull_layout(int nf, int words, int all, size_t base, const CullSpec& 
 // culling tables (256-B aligned): n_images * n_pixels doubles.
 size_t image64_offset(size_t end) { return align256(end); }
 
-// Workspace of an image render through the spot tree: its layout, then the
-// fp64 sums.
-static size_t tree_workspace_bytes(const iact_scene& sc, const TreeLayout& T) {
-  return T.sums + (size_t)sc.sensor.n_pixels * sizeof(double);
-}
-
 // tree: the render takes the spot tree where that serves it
 static size_t workspace_bytes_for(const iact_scene& sc, int ns, int mode, const LaunchShape& shp,
                                   const TraceArgs& A, const DevInfo& dev, bool tree) {
   LaunchShape ts;
-  if (mode == IACT_MODE_IMAGE && tree && tree_serves(A, 0, dev, ts))
-    return tree_workspace_bytes(sc, tree_layout(sc, ns, tree_sorts(A, ns)));
+  if (mode == IACT_MODE_IMAGE && tree && tree_serves(A, 0, 0, dev, ts))
+    return tree_layout(sc, ns, tree_sorts(A, ns), ts.grid).end;
   const size_t base = base_workspace_bytes(sc, mode, shp, A);
   const CullSpec c{ns, 1, nullptr, mode == IACT_MODE_IMAGE && !A.det, refine_groups(A, mode)};
   const size_t end = cull_layout(A.nf, A.cull_words, A.cull_all, base, c).end;
@@ -594,9 +588,8 @@ int adj_sm_layout(const iact_scene& sc, const double* sources, const float* valu
   out.torque = align256(end);
   out.end = out.torque + (size_t)3 * sc.facets.n_facets * sizeof(double);
   LaunchShape ts;
-  if (tree_serves(A, 1, dev, ts)) {
-    const size_t t = tree_layout(sc, ns, tree_sorts(A, ns)).sums +
-                     (size_t)3 * sc.facets.n_facets * sizeof(double);
+  if (tree_serves(A, 1, 0, dev, ts)) {
+    const size_t t = tree_layout(sc, ns, tree_sorts(A, ns), 0).end;
     if (t > out.end) out.end = t;
   }
   return IACT_OK;
@@ -770,18 +763,13 @@ static int32_t trace_fwd(const iact_scene* scene, const double* sources, const f
   hipError_t e = hipSuccess;
   const bool empty = (sc.facets.n_facets == 0 || n_sources == 0);
   LaunchShape tshp;
-  if (mode == IACT_MODE_IMAGE && !empty && want_tree && tree_serves(A, 0, dev, tshp)) {
-    const TreeLayout T = tree_layout(sc, n_sources, tree_sorts(A, n_sources));
+  if (mode == IACT_MODE_IMAGE && !empty && want_tree && tree_serves(A, 0, 0, dev, tshp)) {
+    const TreeLayout T = tree_layout(sc, n_sources, tree_sorts(A, n_sources), tshp.grid);
     AdjArgs B;
     memset(&B, 0, sizeof(B));
     B.T = A;
-    B.T.out64 = (double*)((char*)workspace + T.sums);
-    e = launch_fill_d(B.T.out64, P, 0.0, st);
-    if (e != hipSuccess) return hip_error(e, "clear image sums");
-    rc = launch_tree(B, T, workspace, tshp, source_type, 0, st);
-    if (rc) return rc;
-    e = launch_f64_to_f32(B.T.out64, out, P, st);
-    return e == hipSuccess ? IACT_OK : hip_error(e, "k_f64_to_f32");
+    B.T.partials = (float*)((char*)workspace + T.sums);
+    return launch_tree(B, T, workspace, tshp, source_type, 0, 0, st);
   }
   if (!empty) {
     const CullSpec c{n_sources, 1, nullptr, mode == IACT_MODE_IMAGE && !A.det,

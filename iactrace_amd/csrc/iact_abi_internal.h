@@ -60,18 +60,21 @@ int adj_sm_layout(const iact_scene& sc, const double* sources, const float* valu
                   const iact_launch* L, const DevInfo& dev, TraceArgs& A, LaunchShape& shp,
                   AdjSmLayout& out);
 // The spot tree (iact_tree.hip): workspace (records at 0, then the byte offsets
-// below; `sums` is free for the caller's fp64 sums), node counts per facet.
+// below; `sums`: the blocks' partial images or the facets' torques), node
+// counts per facet.
 struct TreeLayout {
   size_t nodes, balls, frame, table, sws, perm, src, val, sums, end;
   int n_top, n_patch, n_leaf;
   bool sort;
 };
-TreeLayout tree_layout(const iact_scene& sc, int ns, bool sort);
+TreeLayout tree_layout(const iact_scene& sc, int ns, bool sort, int grid);
+int tree_max_grid(const DevInfo& dev);
 // Whether the tree takes this source-major launch (mode 0 image, 1 rotation
-// gradients, 2 all gradients), and its launch shape.
-bool tree_serves(const TraceArgs& A, int mode, const DevInfo& dev, LaunchShape& shp);
+// gradients, 2 all gradients), and its launch shape.  n_acc: fp64 sums that mode
+// 2 keeps per source (1 value gradients, 4 also source gradients, else 0).
+bool tree_serves(const TraceArgs& A, int mode, int n_acc, const DevInfo& dev, LaunchShape& shp);
 int launch_tree(AdjArgs& B, const TreeLayout& T, void* workspace, const LaunchShape& shp,
-                int source_type, int mode, hipStream_t st);
+                int source_type, int mode, int n_acc, hipStream_t st);
 // An image or gradient launch may reorder its sources into direction cells.
 inline bool tree_sorts(const TraceArgs& A, int ns) {
   return A.cull_words > 0 && !A.cull_all && ns >= kChunkCullMinSources;

@@ -677,13 +677,14 @@ int32_t iact_trace_bwd(const iact_scene* scene, const double* sources, const flo
     B.g_src = grads->sources;
     B.g_val = grads->values;
     const int mode = B.g_pos || B.g_src || B.g_val ? 2 : 1;
+    const int n_acc = B.g_src ? 4 : (B.g_val ? 1 : 0);
     LaunchShape tshp;
-    if (tree_serves(A, mode, dev, tshp)) {
-      const TreeLayout T = tree_layout(sc, n_sources, tree_sorts(A, n_sources));
+    if (tree_serves(A, mode, n_acc, dev, tshp)) {
+      const TreeLayout T = tree_layout(sc, n_sources, tree_sorts(A, n_sources), 0);
       B.torque = (double*)((char*)workspace + T.sums);
       e = launch_fill_d(B.torque, 3ll * nf, 0.0, st);
       if (e != hipSuccess) return hip_error(e, "clear torques");
-      rc = launch_tree(B, T, workspace, tshp, source_type, mode, st);
+      rc = launch_tree(B, T, workspace, tshp, source_type, mode, n_acc, st);
       if (rc) return rc;
       if (grads->rotations) {
         e = launch_torque_to_euler(B.torque, sc.facets.rotations, nf, grads->rotations, st);

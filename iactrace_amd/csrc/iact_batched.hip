@@ -180,9 +180,10 @@ static size_t instance_need(const iact_scene* scene, long long ns, int words, in
   const CullSpec c{ns, 1, nullptr, true, (total + 63) / 64};
   const size_t end = cull_layout(scene->facets.n_facets, words, all, recs, c).end;
   const size_t old = image64_offset(end) + (size_t)scene->sensor.n_pixels * sizeof(double);
-  // (the spot tree sorts from kChunkCullMinSources sources of obstructed scenes)
-  const size_t tree = tree_layout(*scene, (int)ns, words > 0).sums +
-                      (size_t)scene->sensor.n_pixels * sizeof(double);
+  // the spot tree: sorted sources and a full grid's partial images at most
+  DevInfo dev;
+  if (device_info(dev)) return old;
+  const size_t tree = tree_layout(*scene, (int)ns, words > 0, tree_max_grid(dev)).end;
   return tree > old ? tree : old;
 }
 

@@ -9,6 +9,7 @@ namespace iact {
 
 struct LaunchShape {
   int grid;
+  int full_grid = 0;  // the spot tree's: the blocks that the GPU holds
   int threads;
   size_t lds;
 };

@@ -61,11 +61,12 @@ struct TreeParams {
   const float* frame;    // reference direction (see k_tree_frame)
   const int16_t* table;  // staged hexagonal table (see k_tree_frame)
   int n_top, n_patch, n_leaf, per_facet;  // nodes per facet
-  uint32_t n_sb, items;                   // source blocks, work items
-  FastDiv d_sb, d_top;                    // divide by n_sb, by n_top
+  uint32_t n_sb, n_part, items;           // source blocks, parts of a top, work items
+  FastDiv d_sb, d_part, d_top;            // divide by n_sb, by n_part, by n_top
   float b0[3], b1[3], b2[3];  // columns of the inverse of the rows (An, Au, Av)
   float n_au, n_av;           // |Au|, |Av|
   float hu, hv;               // half a pixel less the edge, in the test's forms
+  int n_acc;                  // fp64 sums kept per source (gradients)
 };
 
 struct TraceArgs {
@@ -106,7 +107,7 @@ struct TraceArgs {
   int32_t* dbg_pix;
   float* partials;
   const float* world;  // SoA (7, nf*M) when precomputed
-  int lds_image;       // image accumulated in LDS
+  int lds_image;       // image accumulated in LDS: 1 fp32, 2 fp64 (source-major)
   int lds_table;       // hex table staged in LDS
   int det;             // deterministic (wave-private images, ordered sums)
   int max_rounds;
@@ -587,14 +588,14 @@ IACT_DEV float primary_shadow(const TraceArgs& A, const Sample& s, f3 d, bool ac
 // distance of closest approach by up to some 13 2^-24 |oc|^2, so a thin member
 // far away may be hit by rays that pass centimetres off it.
 IACT_DEV float reach_radius(float r, f3 w, float rho) {
-  const float oc = sqrtf(dot(w, w)) + rho;
-  return fmaf(sqrtf(fmaf(1.5e-6f * oc, oc, r * r)), 1.001f, 1e-3f);
+  const float oc = fsqrt(dot(w, w)) + rho;
+  return fmaf(fsqrt(fmaf(1.5e-6f * oc, oc, r * r)), 1.001f, 1e-3f);
 }
 IACT_DEV bool bundle_reaches(f3 c, float rho, f3 a, float tn, f3 b, float R) {
   const f3 w = b - c;
   const float s = dot(w, a);
   const f3 perp = fma3(-s, a, w);
-  const float e = sqrtf(dot(perp, perp));
+  const float e = fsqrt(dot(perp, perp));
   const float rr = reach_radius(R, w, rho) + rho;
   // written so that NaN geometry keeps the candidate
   return !(s + rr < 0.f) && !(e > fmaf(tn, s + rr, rr));
@@ -614,28 +615,33 @@ IACT_DEV bool obstruction_reaches(const iact_obstructions& ob, int j, f3 c, floa
   const int c0 = ob.n_cylinders, c1 = c0 + ob.n_boxes, c2 = c1 + ob.n_spheres;
   const int c3 = c2 + ob.n_oriented_boxes;
   if (j < c0) return cylinder_reaches((Row)(ob.cylinders + 8 * j), c, rho, a, tn);
+  // the bounding sphere (b, R) of the other kinds
+  f3 b;
+  float R;
   if (j < c1) {
     const Row q = (Row)(ob.boxes + 6 * (j - c0));
     const f3 lo = mk3(q[0], q[1], q[2]), hi = mk3(q[3], q[4], q[5]);
     const f3 dd = hi - lo;
-    return bundle_reaches(c, rho, a, tn, 0.5f * (lo + hi), 0.5f * sqrtf(dot(dd, dd)));
-  }
-  if (j < c2) {
+    b = 0.5f * (lo + hi);
+    R = 0.5f * fsqrt(dot(dd, dd));
+  } else if (j < c2) {
     const Row q = (Row)(ob.spheres + 4 * (j - c1));
-    return bundle_reaches(c, rho, a, tn, mk3(q[0], q[1], q[2]), q[3]);
-  }
-  if (j < c3) {
+    b = mk3(q[0], q[1], q[2]);
+    R = q[3];
+  } else if (j < c3) {
     const Row q = (Row)(ob.oriented_boxes + 15 * (j - c2));
     const f3 he = mk3(q[3], q[4], q[5]);
-    return bundle_reaches(c, rho, a, tn, mk3(q[0], q[1], q[2]), sqrtf(dot(he, he)));
+    b = mk3(q[0], q[1], q[2]);
+    R = fsqrt(dot(he, he));
+  } else {
+    const Row q = (Row)(ob.triangles + 9 * (j - c3));
+    const f3 v0 = mk3(q[0], q[1], q[2]), v1 = mk3(q[3], q[4], q[5]);
+    const f3 v2 = mk3(q[6], q[7], q[8]);
+    b = (1.f / 3.f) * (v0 + v1 + v2);
+    const f3 e0 = v0 - b, e1 = v1 - b, e2 = v2 - b;
+    R = fsqrt(fmaxf(fmaxf(dot(e0, e0), dot(e1, e1)), dot(e2, e2)));
   }
-  const Row q = (Row)(ob.triangles + 9 * (j - c3));
-  const f3 v0 = mk3(q[0], q[1], q[2]), v1 = mk3(q[3], q[4], q[5]);
-  const f3 v2 = mk3(q[6], q[7], q[8]);
-  const f3 ctr = (1.f / 3.f) * (v0 + v1 + v2);
-  const f3 e0 = v0 - ctr, e1 = v1 - ctr, e2 = v2 - ctr;
-  const float R = sqrtf(fmaxf(fmaxf(dot(e0, e0), dot(e1, e1)), dot(e2, e2)));
-  return bundle_reaches(c, rho, a, tn, ctr, R);
+  return bundle_reaches(c, rho, a, tn, b, R);
 }
 
 // Can a ray of the bundle reach cylinder q (p1, unit axis, height, radius)?
@@ -659,8 +665,8 @@ IACT_DEV bool cylinder_reaches(Ptr q, f3 c, float rho, f3 a, float tn) {
   // interval of t with s(t) + rr >= 0 and g(t) >= 0
   float lo = 0.f, hi = h;
   auto clip = [&](float k0, float k1) {  // k0 + k1 t >= 0
-    if (k1 > 0.f) lo = fmaxf(lo, -k0 / k1);
-    else if (k1 < 0.f) hi = fminf(hi, -k0 / k1);
+    if (k1 > 0.f) lo = fmaxf(lo, -k0 * frcp(k1));
+    else if (k1 < 0.f) hi = fminf(hi, -k0 * frcp(k1));
     else if (k0 < 0.f) hi = -1.f;
   };
   clip(s0 + rr, s1);
@@ -670,7 +676,7 @@ IACT_DEV bool cylinder_reaches(Ptr q, f3 c, float rho, f3 a, float tn) {
   const float qc = dot(P0, P0) - G0 * G0;
   auto Q = [&](float t) { return fmaf(fmaf(qa, t, qb), t, qc); };
   float m = fminf(Q(lo), Q(hi));
-  if (qa > 0.f) m = fminf(m, Q(fminf(fmaxf(-qb / (2.f * qa), lo), hi)));
+  if (qa > 0.f) m = fminf(m, Q(fminf(fmaxf(-0.5f * qb * frcp(qa), lo), hi)));
   const float hh = fmaxf(fabsf(lo), fabsf(hi));
   const float tol =
       1e-5f * (dot(P0, P0) + G0 * G0 + hh * hh * (dot(P1, P1) + G1 * G1) + 1e-6f);
@@ -684,8 +690,7 @@ IACT_DEV bool cylinder_reaches(Ptr q, f3 c, float rho, f3 a, float tn) {
 // central ray), which is much tighter than its bounding sphere.
 IACT_DEV bool line_reaches(const iact_obstructions& ob, int j, f3 c, float rho, f3 a) {
   const int c0 = ob.n_cylinders, c1 = c0 + ob.n_boxes;
-  if (j < c0) return cylinder_reaches(as_const(ob.cylinders) + 8 * j, c, rho, a, 0.f);
-  if (j >= c1) return obstruction_reaches<true>(ob, j, c, rho, a, 0.f);
+  if (j < c0 || j >= c1) return obstruction_reaches<true>(ob, j, c, rho, a, 0.f);
   const cptr<float> q = as_const(ob.boxes) + 6 * (j - c0);
   const float g = fmaf(rho, 1.001f, 1e-3f + 1e-5f * (fabsf(c.x) + fabsf(c.y) + fabsf(c.z)));
   // (a direction component of 0 as 1e-9: no 0 * inf)

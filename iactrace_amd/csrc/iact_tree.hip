@@ -38,7 +38,7 @@
 
 namespace iact {
 
-constexpr int kWaves = kTreeSources / 64;
+constexpr int kWaves = 8;  // of a block
 constexpr float kTreeEps = 2e-6f;  // margin: some four times the fp32 rounding of a hit
 
 // Node words: 0-1 P, 2-5 Q (u: a, b; v: a, b), 6-7 h, 8-11 J (u: 1, 2; v: 1,
@@ -421,7 +421,7 @@ IACT_DEV void group_node(const TreeParams& K, const SpotSample& s, bool act, flo
 // One block of four waves per (facet, top): a wave per patch of 64 records
 // makes the patch's node and its four leaves' (wave reductions), then the
 // block makes the top's from the patches' moments and a second pass over the
-// samples.  28 us for 875 x 1024 samples: latency and the reductions' VALU.
+// samples.  87 us for 875 x 1024 samples: the reductions' VALU.
 template <int KIND>
 __global__ __launch_bounds__(256) void k_tree_nodes(TraceArgs A, TreeParams K, float* nodes, float* balls) {
   __shared__ float mom[16][36];
@@ -564,26 +564,39 @@ __global__ __launch_bounds__(256) void k_tree_nodes(TraceArgs A, TreeParams K, f
 
 // ------------------------------------------------------------------ walk
 // LDS of a block (byte offsets): the item's sources, the lists and sums at
-// fixed offsets, then the image (or image gradient) behind one spare entry, the
-// staged table and the candidate list.
+// fixed offsets, then the image (fp64, see lds_add) or the image gradient (fp32)
+// behind one spare entry, the staged table, the candidate list with each wave's
+// selection from it, and the per-source gradient sums (fp64: value, then sum G nrwh m).
 template <int MODE>
 struct TreeLds {
+  using Img = std::conditional_t<MODE == 0, double, float>;
   static constexpr uint32_t src = 0;  // e, value / |u|, da, db (, 1 / |u|)
-  static constexpr uint32_t acc = src + (MODE == 2 ? 7u : 6u) * kTreeSources * 4u;
-  static constexpr uint32_t l0 = acc + (MODE == 2 ? 4u : 0u) * kTreeSources * 4u;
+  static constexpr uint32_t l0 = src + (MODE == 2 ? 7u : 6u) * kTreeSources * 4u;
   static constexpr uint32_t wl = l0 + kTreeSources * 2u;
   static constexpr uint32_t pc = wl + kWaves * 2u * kTreeSources * 2u;
   static constexpr uint32_t red = pc + kWaves * 64u * 2u;
   static constexpr uint32_t img = red + 256u;
 };
-IACT_DEV uint32_t tree_tab_offset(uint32_t img, int n_pixels) {
-  return (img + (uint32_t)(n_pixels + 1) * 4u + 15u) & ~15u;
+template <int MODE>
+__host__ __device__ inline uint32_t tree_tab_at(int n_pixels) {
+  return (TreeLds<MODE>::img +
+          (uint32_t)(n_pixels + 1) * (uint32_t)sizeof(typename TreeLds<MODE>::Img) + 15u) &
+         ~15u;
+}
+__host__ __device__ inline uint32_t tree_lc_at(uint32_t tab_at, int table_words) {
+  return (tab_at + (uint32_t)table_words * 2u + 15u) & ~15u;
+}
+__host__ __device__ inline uint32_t tree_gm_at(uint32_t lc_at, int n_ob) {
+  return (lc_at + (uint32_t)n_ob * 2u + 15u) & ~15u;
+}
+__host__ __device__ inline uint32_t tree_acc_at(uint32_t gm_at, int n_ob) {
+  return gm_at + (uint32_t)((n_ob + 63) / 64) * 8u * (uint32_t)kWaves;
 }
 template <int MODE>
-static size_t tree_lds_bytes(int n_pixels, int table_words, int n_ob) {
-  size_t o = (TreeLds<MODE>::img + (size_t)(n_pixels + 1) * 4u + 15u) & ~(size_t)15u;
-  o = (o + (size_t)table_words * 2u + 15u) & ~(size_t)15u;
-  return o + (size_t)n_ob * 2u;
+static size_t tree_lds_bytes(int n_pixels, int table_words, int n_ob, int n_acc) {
+  const uint32_t lc = tree_lc_at(tree_tab_at<MODE>(n_pixels), table_words);
+  return (size_t)tree_acc_at(tree_gm_at(lc, n_ob), n_ob) +
+         (size_t)n_acc * kTreeSources * sizeof(double);
 }
 static int table_words(const DevSensor& S) {
   return S.kind == IACT_SENSOR_HEX ? (S.tq + 4) * (S.tr + 4) : 0;
@@ -651,6 +664,11 @@ IACT_DEV int node_test(const DevSensor& S, const TreeParams& K, const int16_t* t
   return fm < K.hu ? max(code, -1) : (code == -2 && fm < 1.99f ? -1 : kUnresolved);
 }
 
+IACT_DEV int lanes_below(uint64_t mask) {  // set bits below the lane's own
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                   __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
 // Wave-private list in LDS: one list grows from the front, one from the back.
 struct WaveList {
   uint16_t* l;
@@ -658,12 +676,8 @@ struct WaveList {
 };
 IACT_DEV void push(WaveList& w, bool front, bool back, int v) {
   const uint64_t bf = __ballot(front), bb = __ballot(back);
-  const int pf = __builtin_amdgcn_mbcnt_hi((uint32_t)(bf >> 32),
-                                           __builtin_amdgcn_mbcnt_lo((uint32_t)bf, 0u));
-  const int pb = __builtin_amdgcn_mbcnt_hi((uint32_t)(bb >> 32),
-                                           __builtin_amdgcn_mbcnt_lo((uint32_t)bb, 0u));
-  if (front) w.l[w.n + pf] = (uint16_t)v;
-  if (back) w.l[kTreeSources - 1 - (w.m + pb)] = (uint16_t)v;
+  if (front) w.l[w.n + lanes_below(bf)] = (uint16_t)v;
+  if (back) w.l[kTreeSources - 1 - (w.m + lanes_below(bb))] = (uint16_t)v;
   w.n += __popcll(bf);
   w.m += __popcll(bb);
 }
@@ -733,35 +747,47 @@ IACT_DEV uint32_t shade_bits(const iact_obstructions& ob, int j, f3 myp, int nq,
 // patch's leaves and traces what is left there ray by ray -- always 64 pairs
 // per instruction, whatever the fraction that splits.  MODE 0: image; 1:
 // rotation gradients; 2: also positions, values, sources.
+// VALU issue bounds it (82-87 % of the busy cycles), about half in the rays of
+// unresolved leaves.  One ray per (sample, source) took 3693 us for 875 facets
+// x 1024 samples x 4096 sources without obstructions, this 960; 12732 against
+// 4200 us with 122 obstructions and a hexagonal camera, rough mirrors.  Eight
+// waves share one image, so 24 waves and their sources fit a CU; four-wave
+// blocks: 5007 against 4611 us.  Six waves per SIMD for the obstructed
+// gradients: 6.23 against 6.43 ms for the iteration above kWaves' rule; the
+// image kernels need no bound (4528 against 4537 us with one).
 template <int SRC, int KIND, int OBST, int MODE>
-__global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) {
+__global__ __launch_bounds__(64 * kWaves)
+__attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B, TreeParams K) {
   const TraceArgs& A = B.T;
-  constexpr int NS = kTreeSources;
+  constexpr int NS = kTreeSources, NT = 64 * kWaves;
   extern __shared__ __align__(16) char sm[];
   const int P = A.S.n_pixels;
   const int tw = KIND == IACT_SENSOR_HEX ? (A.S.tq + 4) * (A.S.tr + 4) : 0;
   const int n_ob = OBST ? n_obstructions(A.ob) : 0;
   using L = TreeLds<MODE>;
-  float* img = (float*)(sm + L::img) + 1;  // (MODE > 0: the image gradient; [-1] = 0)
-  const uint32_t tab_at = tree_tab_offset(L::img, P);
+  auto* img = (typename L::Img*)(sm + L::img) + 1;  // (MODE > 0: the gradient; [-1] = 0)
+  const uint32_t tab_at = tree_tab_at<MODE>(P), lc_at = tree_lc_at(tab_at, tw);
   int16_t* tab = (int16_t*)(sm + tab_at);
   float* sx = (float*)(sm + L::src);
   float *sy = sx + NS, *sz = sx + 2 * NS, *svi = sx + 3 * NS, *sda = sx + 4 * NS;
   float *sdb = sx + 5 * NS, *sinv = sx + 6 * NS;
-  float* acc = (float*)(sm + L::acc);  // MODE 2: value gradient, then sum G nrwh m
+  const uint32_t gm_at = tree_gm_at(lc_at, n_ob);
+  double* acc = (double*)(sm + tree_acc_at(gm_at, n_ob));  // (MODE 2)
   uint16_t* l0 = (uint16_t*)(sm + L::l0);
-  uint16_t* lc = (uint16_t*)(sm + ((tab_at + (uint32_t)tw * 2u + 15u) & ~15u));
+  uint16_t* lc = (uint16_t*)(sm + lc_at);
   float* red = (float*)(sm + L::red);          // 32 floats
   int* cnt = (int*)(sm + L::red + 128);        // 4 ints
-  double* tot = (double*)(sm + L::red + 144);  // 6 doubles
+  uint32_t& work_next = *(uint32_t*)(sm + L::red + 144);
+  double* tot = (double*)(sm + L::red + 160);  // 6 doubles
   const int tid = threadIdx.x, lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   uint16_t* wl1 = (uint16_t*)(sm + L::wl) + (2 * wave) * NS;
   uint16_t* wl2 = wl1 + NS;
   uint16_t* pc = (uint16_t*)(sm + L::pc) + 64 * wave;
-  if (tid == 0) img[-1] = 0.f;
-  for (int i = tid; i < P; i += NS) img[i] = MODE ? B.grad_image[i] : 0.f;
-  for (int i = tid; i < tw; i += NS) tab[i] = K.table[i];
+  uint64_t* gm = (uint64_t*)(sm + gm_at) + wave * ((n_ob + 63) / 64);
+  if (tid == 0) img[-1] = 0;
+  for (int i = tid; i < P; i += NT) img[i] = MODE ? B.grad_image[i] : 0.f;
+  for (int i = tid; i < tw; i += NT) tab[i] = K.table[i];
   const cptr<float> fr = as_const(K.frame);
   const float a0 = fr[0], b0 = fr[1], tau = fr[2], sign = fr[3];
   const long long total = (long long)A.nf * A.M;
@@ -776,45 +802,51 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
   // one is walked.
   uint32_t* const work = (uint32_t*)K.frame + 4;
   for (uint32_t item = blockIdx.x; item < K.items;) {
-    const uint32_t ft = fdiv(item, K.d_sb);
-    const int sb = (int)(item - ft * K.n_sb);
+    const uint32_t ftp = fdiv(item, K.d_sb);
+    const int sb = (int)(item - ftp * K.n_sb);
+    const uint32_t ft = fdiv(ftp, K.d_part);
+    const int part = (int)(ftp - ft * K.n_part);
     const int f = (int)fdiv(ft, K.d_top), top = (int)ft - f * K.n_top;
     const int npt = (min(kTopSamples, A.M - top * kTopSamples) + 63) / 64;
     const long long nbase = (long long)f * K.per_facet;
     const cptr<float> tnode = as_const(K.nodes) + IACT_NODE_WORDS * (nbase + top);
     const cptr<float> tball = as_const(K.balls) + 4 * (nbase + top);
-    __syncthreads();  // the previous item's lists and sums are done with
-    if (tid < 4) cnt[tid] = tid == 3 ? (int)(gridDim.x + atomicAdd(work, 1u)) : 0;
+    uint32_t next = 0u;  // (thread 0's; used when the item is done)
+    if (tid == 0) next = gridDim.x + atomicAdd(work, 1u);
+    if (tid < 4) cnt[tid] = 0;
     if (MODE && tid < 6) tot[tid] = 0.0;
     if (MODE == 2) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i * NS + tid] = 0.f;
+      for (int i = tid; i < K.n_acc * NS; i += NT) acc[i] = 0.0;
     }
-    // ---- the item's sources, one per thread
-    const int sidx = sb * NS + tid;
-    const bool valid = sidx < A.ns;
-    const int sl = valid ? sidx : A.ns - 1;
+    // ---- the item's sources
     const cptr<float> fp = as_const(A.positions) + 3 * f;
     const f3 pos = mk3(fp[0], fp[1], fp[2]);
-    const double* sp = A.sources + 3 * (size_t)sl;
-    const f3 e = source_offset<SRC>(sp[0], sp[1], sp[2], pos);
-    const float value = valid ? A.values[sl] : 0.f;
-    const float ie = frsq(dot(e, e));
-    const float inv = SRC == IACT_SOURCE_POINT ? ie : 1.f;
-    const float vinv = value * inv;
-    const bool far = valid && (SRC != IACT_SOURCE_POINT || source_qs(A, e) == 0.f);
-    const f3 U = sensor_dirs(A.S, e);
-    const float iu = frcp(U.x);
-    float da = fmaf(U.y, iu, -a0), db = fmaf(U.z, iu, -b0);
-    if (!(far && U.x * ie * sign > 1e-3f && fabsf(da) + fabsf(db) <= tau)) da = __builtin_nanf("");
-    sx[tid] = e.x;
-    sy[tid] = e.y;
-    sz[tid] = e.z;
-    svi[tid] = vinv;
-    sda[tid] = da;
-    sdb[tid] = db;
-    if (MODE == 2) sinv[tid] = inv;
-    const f3 dsh = -(ie * e);  // unit direction towards the source
+    f3 dsum = mk3(0.f, 0.f, 0.f);  // of the unit directions towards them
+#pragma unroll
+    for (int r = 0; r < NS; r += NT) {
+      const int si = r + tid, sidx = sb * NS + si;
+      const bool valid = sidx < A.ns;
+      const int sl = valid ? sidx : A.ns - 1;
+      const double* sp = A.sources + 3 * (size_t)sl;
+      const f3 e = source_offset<SRC>(sp[0], sp[1], sp[2], pos);
+      const float value = valid ? A.values[sl] : 0.f;
+      const float ie = frsq(dot(e, e)), inv = SRC == IACT_SOURCE_POINT ? ie : 1.f;
+      const bool far = valid && (SRC != IACT_SOURCE_POINT || source_qs(A, e) == 0.f);
+      const f3 U = sensor_dirs(A.S, e);
+      const float iu = frcp(U.x);
+      float da = fmaf(U.y, iu, -a0);
+      const float db = fmaf(U.z, iu, -b0);
+      if (!(far && U.x * ie * sign > 1e-3f && fabsf(da) + fabsf(db) <= tau))
+        da = __builtin_nanf("");
+      sx[si] = e.x;
+      sy[si] = e.y;
+      sz[si] = e.z;
+      svi[si] = value * inv;
+      sda[si] = da;
+      sdb[si] = db;
+      if (MODE == 2) sinv[si] = inv;
+      if (OBST && valid) dsum = dsum - ie * e;
+    }
     // ---- obstruction candidates of the item: those the cone of its sources'
     // directions (with the parallax of near ones) can reach from the top's ball
     const f3 tc = mk3(tball[0], tball[1], tball[2]);
@@ -822,8 +854,7 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
     f3 ax = mk3(0.f, 0.f, 1.f);
     float tn = -1.f;
     if (OBST && !A.cull_all) {
-      const f3 w = valid ? dsh : mk3(0.f, 0.f, 0.f);
-      const float wx = wave_sum(w.x), wy = wave_sum(w.y), wz = wave_sum(w.z);
+      const float wx = wave_sum(dsum.x), wy = wave_sum(dsum.y), wz = wave_sum(dsum.z);
       if (lane == 0) {
         red[3 * wave] = wx;
         red[3 * wave + 1] = wy;
@@ -836,37 +867,44 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
         sum = sum + mk3(red[3 * i], red[3 * i + 1], red[3 * i + 2]);
       const float la = dot(sum, sum);
       if (la > 0.f) ax = frsq(la) * sum;
-      float ang = 0.f;
-      if (valid) {
-        // (from the chord: acos of a cosine next to 1 is off by 3e-4 rad)
-        const f3 ch = dsh - ax;
-        ang = 2.f * asinf(fminf(0.5f * sqrtf(dot(ch, ch)), 1.f));
-        if (SRC == IACT_SOURCE_POINT)
-          ang += trho * ie < 1.f ? asinf(trho * ie) : 3.1415927f;
-        if (!(ang >= 0.f)) ang = 3.1415927f;  // NaN: no culling
+      // the largest tan(angle + parallax), from the chord (acos of a cosine
+      // next to 1 would be off by 3e-4 rad); beyond 80 degrees: no culling
+      float tg = 0.f;
+#pragma unroll
+      for (int r = 0; r < NS; r += NT) {
+        const int si = r + tid;
+        const f3 e = mk3(sx[si], sy[si], sz[si]);
+        const float ie = frsq(dot(e, e));
+        const f3 ch = -ie * e - ax;
+        const float c2 = dot(ch, ch), cs = fmaf(-0.5f, c2, 1.f);
+        float g = cs > 0.17f ? fsqrt(c2 * fmaf(-0.25f, c2, 1.f)) * frcp(cs) : 1e30f;
+        if (SRC == IACT_SOURCE_POINT) {
+          const float sp = trho * ie, cp2 = fmaf(-sp, sp, 1.f);
+          const float tp = cp2 > 0.03f ? sp * frsq(cp2) : 1e30f;
+          g = g * tp < 0.9f ? (g + tp) * frcp(fmaf(-g, tp, 1.f)) : 1e30f;
+        }
+        if (!(g < 5.6f)) g = 1e30f;  // (NaN too)
+        if (sb * NS + si < A.ns) tg = fmaxf(tg, g);
       }
-      ang = group_max<64>(ang);
-      if (lane == 0) red[24 + wave] = ang;
+      tg = group_max<64>(tg);
+      if (lane == 0) red[24 + wave] = tg;
       __syncthreads();
 #pragma unroll
-      for (int i = 0; i < kWaves; ++i) ang = fmaxf(ang, red[24 + i]);
-      const float th = ang + 2e-4f;
-      tn = th < 1.4f ? tanf(th) : -1.f;
+      for (int i = 0; i < kWaves; ++i) tg = fmaxf(tg, red[24 + i]);
+      // + 2e-4 rad
+      tn = tg < 5.6f ? fmaf(1.0001f, tg, 2e-4f) * frcp(fmaf(-2e-4f, tg, 1.f)) : -1.f;
     } else {
       __syncthreads();
     }
     if (OBST) {
-      for (int j0 = 0; j0 < n_ob; j0 += NS) {
+      for (int j0 = 0; j0 < n_ob; j0 += NT) {
         const int j = j0 + tid;
         const bool keep = j < n_ob && (tn < 0.f || obstruction_reaches(A.ob, j, tc, trho, ax, tn));
         const uint64_t bk = __ballot(keep);
         int at = 0;
         if (lane == 0 && bk) at = atomicAdd(cnt + 2, __popcll(bk));
         at = __builtin_amdgcn_readfirstlane(at);
-        if (keep)
-          lc[at + __builtin_amdgcn_mbcnt_hi((uint32_t)(bk >> 32),
-                                            __builtin_amdgcn_mbcnt_lo((uint32_t)bk, 0u))] =
-              (uint16_t)j;
+        if (keep) lc[at + lanes_below(bk)] = (uint16_t)j;
       }
       __syncthreads();
     }
@@ -951,48 +989,57 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
         Gp = mk3(0.f, 0.f, 0.f);
       }
     };
-    // ---- the top, one source per thread
-    {
+    // ---- the top
+#pragma unroll
+    for (int r = 0; r < NS; r += NT) {
+      const int si = r + tid;
+      const bool valid = sb * NS + si < A.ns;
+      const f3 e = mk3(sx[si], sy[si], sz[si]);
+      const bool far = valid && (SRC != IACT_SOURCE_POINT || source_qs(A, e) == 0.f);
       bool sus = false;
       if (OBST && nlc > 0) {
         if (nlc <= 64 && !A.cull_all) {
           const int id = lane < nlc ? lc[lane] : 0;
-          sus = reached(nlc == 64 ? ~0ull : (1ull << nlc) - 1ull, id, tc, trho, dsh, far);
+          sus = reached(nlc == 64 ? ~0ull : (1ull << nlc) - 1ull, id, tc, trho,
+                        -(frsq(dot(e, e)) * e), far);
         } else {
           sus = true;
         }
       }
       int code = kUnresolved;
-      if (tnode[31] != 0.f) code = node_test<KIND>(A.S, K, tab, tnode, da, db);
+      if (tnode[31] != 0.f) code = node_test<KIND>(A.S, K, tab, tnode, sda[si], sdb[si]);
       // (a suspect that misses the camera needs no shadow test)
       if (!far || (sus && code != -1)) code = kUnresolved;
-      if (code >= 0) add_pair(tnode, code, e, vinv, tid);
-      end_node(tnode);
-      const uint64_t bf = __ballot(far && code == kUnresolved), bn = __ballot(valid && !far);
+      if (code >= 0 && part == 0) add_pair(tnode, code, e, svi[si], si);
+      const bool split = far && code == kUnresolved, near = valid && !far;
+      const uint64_t bf = __ballot(split), bn = __ballot(near);
       int at = 0;
       if (lane == 0) {
         if (bf) at = atomicAdd(cnt, __popcll(bf));
         if (bn) at |= atomicAdd(cnt + 1, __popcll(bn)) << 16;
       }
       at = __builtin_amdgcn_readfirstlane(at);
-      if ((bf >> lane) & 1ull)
-        l0[(at & 0xffff) + __builtin_amdgcn_mbcnt_hi((uint32_t)(bf >> 32),
-                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)bf, 0u))] =
-            (uint16_t)tid;
-      if ((bn >> lane) & 1ull)
-        l0[NS - 1 - (at >> 16) -
-           __builtin_amdgcn_mbcnt_hi((uint32_t)(bn >> 32),
-                                     __builtin_amdgcn_mbcnt_lo((uint32_t)bn, 0u))] = (uint16_t)tid;
-      flush();
+      if (split) l0[(at & 0xffff) + lanes_below(bf)] = (uint16_t)si;
+      if (near) l0[NS - 1 - (at >> 16) - lanes_below(bn)] = (uint16_t)si;
     }
+    end_node(tnode);
+    flush();
     __syncthreads();
     const int n0 = __builtin_amdgcn_readfirstlane(cnt[0]);
     const int nn = __builtin_amdgcn_readfirstlane(cnt[1]);
-    // ---- patches (and, where there are fewer patches than waves, segments of
-    // the list)
-    const int nseg = n0 + nn == 0 ? 0 : (npt >= 8 ? 1 : (npt >= 4 ? 2 : (npt >= 2 ? 4 : 8)));
-    for (int un = wave; un < npt * nseg; un += kWaves) {
-      const int p = un / nseg, seg = un - p * nseg;
+    // ---- patches (and, where there are few patches for the waves, segments of
+    // the list), taken by the waves one by one
+    const int p0 = (npt * part) / (int)K.n_part, p1 = (npt * (part + 1)) / (int)K.n_part;
+    const int np1 = p1 - p0;
+    const int lseg = np1 >= kWaves ? 0 : (2 * np1 >= kWaves ? 1 : 2);
+    const int nseg = 1 << lseg, nun = n0 + nn == 0 ? 0 : (p1 - p0) << lseg;
+    auto take = [&]() {
+      int u = 0;
+      if (lane == 0) u = atomicAdd(cnt + 3, 1);
+      return __builtin_amdgcn_readfirstlane(u);
+    };
+    for (int un = take(); un < nun; un = take()) {
+      const int p = p0 + (un >> lseg), seg = un & (nseg - 1);
       const int patch = top * (kTopSamples / 64) + p;
       const int mp = patch * 64, np = min(64, A.M - mp), nleaf = (np + 15) / 16;
       const int jp = f * A.M + mp;  // first record
@@ -1001,20 +1048,27 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
       const long long lid0 = nbase + K.n_top + K.n_patch + 4 * patch;
       const f3 bc = mk3(pball[0], pball[1], pball[2]);
       const float brho = pball[3];
-      // the patch's candidates, one per lane of a group of 64 (rarely more than
-      // one group; pid and pmask are those of the group last loaded)
+      // the patch's candidates: groups of 64 of the item's list (rarely more
+      // than one), one per lane, selected by a mask (kept in LDS)
       const int ngrp = OBST ? (nlc + 63) >> 6 : 0;
+      bool cand = false;
+      for (int g = 0; g < ngrp; ++g) {
+        const int i = 64 * g + lane;
+        const uint64_t mk =
+            __ballot(i < nlc && (tn < 0.f || obstruction_reaches(A.ob, lc[min(i, nlc - 1)], bc,
+                                                                 brho, ax, tn)));
+        if (lane == 0) gm[g] = mk;
+        cand |= mk != 0ull;
+      }
+      if (OBST) wave_lds_fence();
       int pid = 0;
       uint64_t pmask = 0ull;
       auto load_group = [&](int g) {
-        const int i = 64 * g + lane;
-        pid = i < nlc ? lc[i] : 0;
-        pmask = __ballot(i < nlc &&
-                         (tn < 0.f || obstruction_reaches(A.ob, pid, bc, brho, ax, tn)));
-        return pmask != 0ull;
+        pid = lc[min(64 * g + lane, nlc - 1)];
+        const uint64_t mk = gm[g];
+        pmask = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)mk) |
+                (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(mk >> 32)) << 32;
       };
-      bool cand = false;
-      for (int g = ngrp - 1; g >= 0; --g) cand |= load_group(g);
 
       // the gradients of a lane's rays of one source, N = sum G nrwh m
       auto add_rays = [&](f3 N, f3 u, float vi, int si) {
@@ -1033,16 +1087,19 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
       // Rays of listed pairs, with the per-ray kernels' arithmetic: ns samples
       // from record j0.  Full waves: lane = source, the records one after
       // another in scalar registers, pixel runs as in k_trace_sm.  A rest of at
-      // most 40 pairs: lane = (source of four, sample of sixteen), the records
-      // in vector registers (some 75 instructions for 64 rays against 40, but
-      // no idle lanes).  BITS: shadow bits per pair (short lists, second form).
+      // most 48 pairs: the wave is 4 SPL sources times 16 / SPL parts of sixteen
+      // samples, SPL records per lane in vector registers, so a short list
+      // fills the lanes.  BITS: shadow bits per pair (short lists, second form).
+      // SPL: four took 1050 us against 1163 with one (and fewer adds per ray)
+      // without obstructions; beside the shadow code four spills the waves'
+      // occupancy (7004 us with obstructions, 4359 with two, 4528 with one).
       auto trace_far = [&](auto gen, auto bits_t, const uint16_t* list, const uint16_t* bits,
                            int n, int j0, int ns) {
         constexpr bool GEN = decltype(gen)::value;
         constexpr bool BITS = decltype(bits_t)::value;
         int done = 0;
         if (!BITS) {
-          for (; n - done > 40; done += 64) {
+          for (; n - done > 48; done += 64) {
             const bool act = done + lane < n;
             const int si = list[act ? done + lane : done];
             const f3 u = mk3(sx[si], sy[si], sz[si]);
@@ -1081,74 +1138,54 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
           }
           if (done >= n) return;
         }
-        const int r = lane & 15, eo = lane >> 4;
+        constexpr int SPL = !OBST ? 4 : MODE == 0 ? 2 : 1, SRCS = 4 * SPL;
+        const int part = lane / SRCS, slot = lane % SRCS;
+#pragma unroll 1
         for (int q = 0; q < ns; q += 16) {
-          const bool in = q + r < ns;
-          const float4* rp = (const float4*)A.recs + 4 * (size_t)(j0 + (in ? q + r : q));
-          const Sample s = unpack_record(RecRaw{rp[0], rp[1], rp[2], rp[3]});
-          // the next pair's source is read while one is traced
-          int at = min(done + eo, n - 1);
-          int si = list[at];
-          f3 u = mk3(sx[si], sy[si], sz[si]);
-          float vi = svi[si];
-          uint32_t sb = BITS ? bits[at] : 0u;
-          for (int k = done; k < n; k += 4) {
-            const bool act = in && k + eo < n;
-            const int sc = si;
-            const f3 uc = u;
-            const float vc = vi;
-            const bool lit = !BITS || !((sb >> r) & 1u);
-            at = min(k + 4 + eo, n - 1);
-            si = list[at];
-            if (BITS) sb = bits[at];
-            const float i1 = SRC == IACT_SOURCE_POINT ? frsq(dot(uc, uc)) : 1.f;
-            const float cu = dot(uc, s.m);
-            float gu, gv;
-            const bool ok = grid_hit<GEN>(s.G, s.N, sensor_dirs(A.S, uc), cu, gu, gv, i1);
-            const int pix = tree_pixel<KIND, GEN>(A.S, tab, gu, gv, ok && act && lit);
-            u = mk3(sx[si], sy[si], sz[si]);
-            vi = svi[si];
-            if (MODE == 0) {
-              // the sixteen rays of a source mostly meet one or two pixels:
-              // those of the first lane's are summed before the add
-              const float v = pix >= 0 ? vc * (cu * s.nrwh) : 0.f;
-              const int p0 = __shfl(pix, lane & 48, 64);
-              const float t = group_sum<16>(pix == p0 ? v : 0.f);
-              const bool own = r == 0 || (pix >= 0 && pix != p0);
-              if (own) lds_add(img + (r == 0 ? p0 : pix), r == 0 ? t : v);
-            } else {
-              const float gn = img[pix] * s.nrwh, w = gn * vc;
-              Aw = fma3(w, uc, Aw);
-              if (MODE == 2) {
-                if (want_pos && SRC == IACT_SOURCE_POINT) {
-                  w1 += w;
-                  Dw = fma3(w * cu * (i1 * i1), uc, Dw);
+          // (samples past the end of the run are its last one again, dropped)
+          Sample smp[SPL];
+          const int sm0 = q + SPL * part;
+#pragma unroll
+          for (int k = 0; k < SPL; ++k) {
+            const float4* rp = (const float4*)A.recs + 4 * (size_t)(j0 + min(sm0 + k, ns - 1));
+            smp[k] = unpack_record(RecRaw{rp[0], rp[1], rp[2], rp[3]});
+          }
+#pragma unroll 1
+          for (int i = done; i < n; i += SRCS) {
+            const int at = min(i + slot, n - 1);
+            const int si = list[at];
+            const uint32_t drop = (BITS ? (uint32_t)bits[at] >> (SPL * part) : 0u) |
+                                  (i + slot < n ? ~0u << min(max(ns - sm0, 0), SPL) : ~0u);
+            const f3 u = mk3(sx[si], sy[si], sz[si]);
+            const float vi = svi[si];
+            const f3 Ud = sensor_dirs(A.S, u);
+            const float rs = SRC == IACT_SOURCE_POINT ? frsq(dot(u, u)) : 1.f;
+            int run_pix = -1;
+            float run_l = 0.f;
+            f3 N = mk3(0.f, 0.f, 0.f);
+#pragma unroll
+            for (int k = 0; k < SPL; ++k) {
+              const Sample& s = smp[k];
+              const float cu = dot(u, s.m);
+              float gu, gv;
+              const bool ok = grid_hit<GEN>(s.G, s.N, Ud, cu, gu, gv, rs);
+              const int pix = tree_pixel<KIND, GEN>(A.S, tab, gu, gv,
+                                                    ok & (((drop >> k) & 1u) == 0u));
+              if (MODE == 0) {
+                if (pix != run_pix) {
+                  if (k > 0) lds_add(img + run_pix, vi * run_l);
+                  run_pix = pix;
+                  run_l = 0.f;
                 }
-                if (want_val) {
-                  const float t = group_sum<16>(gn * (cu * i1));
-                  if (r == 0 && act) lds_add(acc + sc, t);
-                }
-                if (want_src) {
-                  const float tx = group_sum<16>(gn * s.m.x), ty = group_sum<16>(gn * s.m.y);
-                  const float tz = group_sum<16>(gn * s.m.z);
-                  if (r == 0 && act) {
-                    lds_add(acc + NS + sc, tx);
-                    lds_add(acc + 2 * NS + sc, ty);
-                    lds_add(acc + 3 * NS + sc, tz);
-                  }
-                }
+                run_l = fmaf(cu, s.nrwh, run_l);
+              } else {
+                N = fma3(img[pix] * s.nrwh, s.m, N);
               }
             }
-          }
-          if (MODE) {
-            // the lane's rays share m: torque m x sum w u
-            T = T + cross(s.m, Aw);
-            Aw = mk3(0.f, 0.f, 0.f);
-            if (MODE == 2) {
-              Gp = Gp + fma3(w1, s.m, mk3(-Dw.x, -Dw.y, -Dw.z));
-              Dw = mk3(0.f, 0.f, 0.f);
-              w1 = 0.f;
-            }
+            if (MODE == 0)
+              lds_add(img + run_pix, vi * run_l);
+            else
+              add_rays(N, u, vi, si);
           }
         }
       };
@@ -1172,7 +1209,7 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
             if (OBST && cand) {
               const f3 dn = -(frsq(dot(u, u)) * u);
               for (int g = 0; g < ngrp; ++g) {
-                if (ngrp > 1) load_group(g);
+                load_group(g);
                 sus |= pmask != 0ull && (A.cull_all || reached(pmask, pid, bc, brho, dn, act));
               }
             }
@@ -1230,7 +1267,7 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
           const f3 ds = SRC == IACT_SOURCE_POINT ? dn : -u;  // as the per-ray tests have it
           uint64_t pm = 0ull, um = 0ull;  // the lane's, the wave's candidates
           auto patch_group = [&](int g) {
-            if (ngrp > 1) load_group(g);
+            load_group(g);
             pm = um = 0ull;
             for (uint64_t b = pmask; b != 0ull;) {
               const int k = __builtin_ctzll(b);
@@ -1242,7 +1279,6 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
               um |= __any(r) ? 1ull << k : 0ull;
             }
           };
-          if (ngrp == 1) patch_group(0);
           for (int q = 0; q < nleaf; ++q) {
             const cptr<float> lnode = as_const(K.nodes) + IACT_NODE_WORDS * (lid0 + q);
             const cptr<float> lb = as_const(K.balls) + 4 * (lid0 + q);
@@ -1258,7 +1294,7 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
             const uint32_t all = (1u << nq) - 1u;
             uint32_t bits = 0u;
             for (int g = 0; g < ngrp; ++g) {
-              if (ngrp > 1) patch_group(g);
+              if (ngrp > 1 || q == 0) patch_group(g);
               uint64_t lm = um;
               if (!A.cull_all)
                 lm &= __ballot(((um >> lane) & 1ull) &&
@@ -1333,9 +1369,8 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
             float sh = 1.f;
             if (OBST && cand) {
               for (int g = 0; g < ngrp; ++g) {
-                const int id = ngrp == 1 ? pid : lc[min(64 * g + lane, nlc - 1)];
-                const uint64_t mk = ngrp == 1 ? pmask : (nlc - 64 * g >= 64 ? ~0ull : (1ull << (nlc - 64 * g)) - 1ull);
-                sh *= shadow_factor_list(A.ob, id, mk, s.p, -d, act);
+                if (ngrp > 1 || j == 0) load_group(g);
+                sh *= shadow_factor_list(A.ob, pid, pmask, s.p, -d, act);
               }
             }
             float gu, gv;
@@ -1377,44 +1412,72 @@ __global__ __launch_bounds__(kTreeSources) void k_tree(AdjArgs B, TreeParams K) 
       }
       flush();
     }
+    if (tid == 0) work_next = next;
+    __syncthreads();
     if (MODE) {
-      __syncthreads();
-      if (tid < 3 && (tot[tid] != 0.0)) unsafeAtomicAdd(B.torque + 3 * f + tid, tot[tid]);
+      if (tid < 3 && tot[tid] != 0.0) unsafeAtomicAdd(B.torque + 3 * f + tid, tot[tid]);
       if (want_pos && tid < 3 && tot[3 + tid] != 0.0)
         unsafeAtomicAdd(B.g_pos + 3 * f + tid, tot[3 + tid]);
-      if (MODE == 2 && valid && (want_val || want_src)) {
-        const long long so = B.src_perm ? (long long)B.src_perm[sidx] : (long long)sidx;
-        const float gv = acc[tid];
-        if (want_val && gv != 0.f) unsafeAtomicAdd(B.g_val + so, (double)gv);
-        if (want_src) {
-          const f3 N = mk3(acc[NS + tid], acc[2 * NS + tid], acc[3 * NS + tid]);
-          // far: dL/dsrc = -value / |u| (N - (d.N) d); near sources have theirs
-          // summed already; parallel: value N
-          const f3 d = inv * e;
-          const f3 g = SRC == IACT_SOURCE_POINT
-                           ? (far ? (-vinv) * fma3(-dot(d, N), d, N) : N)
-                           : value * N;
-          unsafeAtomicAdd(B.g_src + 3 * so, (double)g.x);
-          unsafeAtomicAdd(B.g_src + 3 * so + 1, (double)g.y);
-          unsafeAtomicAdd(B.g_src + 3 * so + 2, (double)g.z);
-        }
+    }
+    for (int r = 0; (want_val || want_src) && r < NS; r += NT) {
+      const int si = r + tid, sidx = sb * NS + si;
+      if (sidx >= A.ns) break;
+      const long long so = B.src_perm ? (long long)B.src_perm[sidx] : (long long)sidx;
+      if (want_val && acc[si] != 0.0) unsafeAtomicAdd(B.g_val + so, acc[si]);
+      if (want_src) {
+        const f3 N = mk3((float)acc[NS + si], (float)acc[2 * NS + si], (float)acc[3 * NS + si]);
+        const f3 e = mk3(sx[si], sy[si], sz[si]), d = sinv[si] * e;
+        // far: dL/dsrc = -value / |u| (N - (d.N) d); near sources have theirs
+        // summed already; parallel: value N (1 / |u| is 1)
+        const f3 g = SRC == IACT_SOURCE_POINT
+                         ? (source_qs(A, e) == 0.f ? (-svi[si]) * fma3(-dot(d, N), d, N) : N)
+                         : svi[si] * N;
+        unsafeAtomicAdd(B.g_src + 3 * so, (double)g.x);
+        unsafeAtomicAdd(B.g_src + 3 * so + 1, (double)g.y);
+        unsafeAtomicAdd(B.g_src + 3 * so + 2, (double)g.z);
       }
     }
-    item = (uint32_t)__builtin_amdgcn_readfirstlane(cnt[3]);
+    item = __builtin_amdgcn_readfirstlane(work_next);
+    if (MODE) __syncthreads();  // (the sums above are read before they are cleared)
   }
   if (MODE == 0) {
     __syncthreads();
-    for (int i = tid; i < P; i += NS) {
-      const float v = img[i];
-      if (v != 0.f) unsafeAtomicAdd(A.out64 + i, (double)v);
+    float* part = A.partials + (size_t)blockIdx.x * P;
+    for (int i = tid; i < P; i += NT) part[i] = (float)img[i];
+  }
+}
+
+// The image from the blocks' partial images, summed in fp64: one block per 64
+// pixels, a wave per sixteenth of the partials.
+__global__ __launch_bounds__(1024) void k_sum_partials(const float* part, int n, int P,
+                                                       float* out) {
+  __shared__ double red[16][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i = blockIdx.x * 64 + lane;
+  double s = 0.0;
+  if (i < P) {
+    int b = w;
+    for (; b + 112 < n; b += 128) {  // eight loads in flight
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = part[(size_t)(b + 16 * k) * P + i];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s += (double)v[k];
     }
+    for (; b < n; b += 16) s += (double)part[(size_t)b * P + i];
+  }
+  red[w][lane] = s;
+  __syncthreads();
+  if (w == 0 && i < P) {
+    for (int k = 1; k < 16; ++k) s += red[k][lane];
+    out[i] = (float)s;
   }
 }
 
 // ------------------------------------------------------------------ host
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-TreeLayout tree_layout(const iact_scene& sc, int ns, bool sort) {
+TreeLayout tree_layout(const iact_scene& sc, int ns, bool sort, int grid) {
   const int nf = sc.facets.n_facets, M = sc.facets.n_samples;
   TreeLayout T;
   memset(&T, 0, sizeof(T));
@@ -1446,23 +1509,29 @@ TreeLayout tree_layout(const iact_scene& sc, int ns, bool sort) {
     o = align256(o + (size_t)ns * sizeof(float));
   }
   T.sums = o;
-  T.end = o;
+  // the blocks' partial images, or the facets' torques
+  const size_t img = (size_t)grid * sc.sensor.n_pixels * sizeof(float);
+  const size_t tq = (size_t)3 * nf * sizeof(double);
+  T.end = o + (img > tq ? img : tq);
   return T;
 }
 
-bool tree_serves(const TraceArgs& A, int mode, const DevInfo& dev, LaunchShape& shp) {
+// Blocks of a full grid (24 waves per CU).
+int tree_max_grid(const DevInfo& dev) { return dev.n_cu * (24 / kWaves); }
+
+bool tree_serves(const TraceArgs& A, int mode, int n_acc, const DevInfo& dev, LaunchShape& shp) {
   if (A.layout != 2 || A.S.splat || A.n_stages > 0 || A.det || A.nf <= 0 || A.ns <= 0) return false;
   if (A.S.n_pixels > 32767) return false;
   const int n_ob = n_obstructions(A.ob);
   if (n_ob > 65535) return false;
   const int tw = table_words(A.S);
-  const size_t lds = mode == 0   ? tree_lds_bytes<0>(A.S.n_pixels, tw, n_ob)
-                     : mode == 1 ? tree_lds_bytes<1>(A.S.n_pixels, tw, n_ob)
-                                 : tree_lds_bytes<2>(A.S.n_pixels, tw, n_ob);
+  const size_t lds = mode == 0   ? tree_lds_bytes<0>(A.S.n_pixels, tw, n_ob, 0)
+                     : mode == 1 ? tree_lds_bytes<1>(A.S.n_pixels, tw, n_ob, 0)
+                                 : tree_lds_bytes<2>(A.S.n_pixels, tw, n_ob, n_acc);
   if (lds > 65536) return false;
   const long long items = (long long)A.nf * ((A.M + kTopSamples - 1) / kTopSamples) *
                           ((A.ns + kTreeSources - 1) / kTreeSources);
-  if (items >= (1ll << 31)) return false;
+  if (items >= (1ll << 27)) return false;
   // the rows (An, Au, Av) must be invertible (they are for a rotation)
   const f3 n = A.S.An, u = A.S.Au, v = A.S.Av;
   const double det = (double)n.x * ((double)u.y * v.z - (double)u.z * v.y) -
@@ -1472,15 +1541,17 @@ bool tree_serves(const TraceArgs& A, int mode, const DevInfo& dev, LaunchShape& 
                       sqrt((double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z);
   if (!(fabs(det) > 1e-2 * size) || !isfinite(size) || !(size > 0.0)) return false;
   // as many blocks as the CUs hold (160 KB of LDS each)
-  const int held = (int)fmin(3.0, floor(163840.0 / (double)lds));
+  const int held = (int)fmin(24.0 / kWaves, floor(163840.0 / (double)lds));
   long long grid = (long long)dev.n_cu * held;
-  shp.threads = kTreeSources;
+  shp.threads = 64 * kWaves;
   shp.lds = lds;
-  shp.grid = (int)(items < grid ? items : grid);
+  shp.full_grid = (int)grid;
+  // (items may be split into up to 16 parts)
+  shp.grid = (int)(16 * items < grid ? 16 * items : grid);
   return true;
 }
 
-static TreeParams tree_args(TraceArgs& A, const TreeLayout& T, void* workspace) {
+static TreeParams tree_args(TraceArgs& A, const TreeLayout& T, void* workspace, int full_grid) {
   char* ws = (char*)workspace;
   TreeParams K;
   A.recs = (const float*)ws;
@@ -1493,8 +1564,19 @@ static TreeParams tree_args(TraceArgs& A, const TreeLayout& T, void* workspace) 
   K.n_leaf = T.n_leaf;
   K.per_facet = T.n_top + T.n_patch + T.n_leaf;
   K.n_sb = (uint32_t)((A.ns + kTreeSources - 1) / kTreeSources);
-  K.items = (uint32_t)A.nf * (uint32_t)T.n_top * K.n_sb;
+  // Items cost up to some 400 us (a block of sources on the camera against
+  // 1024 samples), so a launch of few of them is split by patches until every
+  // block has six: an iteration over 5 pointings of 1000 sources against 875
+  // facets of 1024 samples (1750 items per launch) takes 7.16 ms with whole
+  // tops and 6.92 ms in parts.  Parts repeat the top's tests, so no more.
+  const uint32_t whole = (uint32_t)A.nf * (uint32_t)T.n_top * K.n_sb;
+  const int most = T.n_patch < 16 ? T.n_patch : 16;
+  K.n_part = 1;
+  while (2 * K.n_part <= (uint32_t)most && (uint64_t)whole * K.n_part < 6ull * (uint64_t)full_grid)
+    K.n_part *= 2;
+  K.items = whole * K.n_part;
   K.d_sb = make_fastdiv(K.n_sb);
+  K.d_part = make_fastdiv(K.n_part);
   K.d_top = make_fastdiv((uint32_t)T.n_top);
   const double r[3][3] = {{A.S.An.x, A.S.An.y, A.S.An.z},
                           {A.S.Au.x, A.S.Au.y, A.S.Au.z},
@@ -1538,10 +1620,11 @@ static const void* pick_tree(const TraceArgs& A, int mode) {
 // The whole trace: sorted sources in obstructed scenes (an item's sources then
 // bound a narrow bundle), frame, records, nodes, walk.
 int launch_tree(AdjArgs& B, const TreeLayout& T, void* workspace, const LaunchShape& shp,
-                int source_type, int mode, hipStream_t st) {
+                int source_type, int mode, int n_acc, hipStream_t st) {
   TraceArgs& A = B.T;
   char* ws = (char*)workspace;
-  TreeParams K = tree_args(A, T, workspace);
+  TreeParams K = tree_args(A, T, workspace, shp.full_grid);
+  K.n_acc = n_acc;
   hipError_t e;
   if (T.sort) {
     int32_t* pm = (int32_t*)(ws + T.perm);
@@ -1579,8 +1662,16 @@ int launch_tree(AdjArgs& B, const TreeLayout& T, void* workspace, const LaunchSh
                  : pick_tree<IACT_SOURCE_PARALLEL, IACT_SENSOR_SQUARE>(A, mode));
   AdjArgs b = B;
   void* args[] = {&b, &K};
-  e = hipLaunchKernel(k, dim3(shp.grid), dim3(shp.threads), args, shp.lds, st);
-  return e == hipSuccess ? IACT_OK : hip_error(e, "k_tree");
+  const int grid = (int)min((uint32_t)shp.grid, K.items);
+  e = hipLaunchKernel(k, dim3(grid), dim3(shp.threads), args, shp.lds, st);
+  if (e != hipSuccess) return hip_error(e, "k_tree");
+  if (mode == 0) {
+    hipLaunchKernelGGL(k_sum_partials, dim3((A.S.n_pixels + 63) / 64), dim3(1024), 0, st,
+                       A.partials, grid, A.S.n_pixels, A.out);
+    e = hipGetLastError();
+    if (e != hipSuccess) return hip_error(e, "k_sum_partials");
+  }
+  return IACT_OK;
 }
 
 }  // namespace iact

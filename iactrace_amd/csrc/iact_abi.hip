@@ -264,7 +264,13 @@ void fill_trace_args(TraceArgs& A, const iact_scene& sc, const double* sources,
   for (int i = 0; i < sc.n_stages; ++i) A.stages[i] = sc.stages[i];
   A.mirrors = sc.mirrors;
   A.n_surfaces = sc.n_surfaces;
-  for (int i = 0; i < sc.n_surfaces; ++i) A.surfaces[i] = sc.surfaces[i];
+  for (int i = 0; i < sc.n_surfaces; ++i) {
+    const iact_surface& su = sc.surfaces[i];
+    A.surfaces[i] = su;
+    bool conic = true;
+    for (int k = 0; k < su.n_aspheric; ++k) conic = conic && su.aspheric[k] == 0.f;
+    A.conic_surfaces |= conic ? 1u << i : 0u;
+  }
   A.ob = sc.obstructions;
   A.S = make_dev_sensor(sc.sensor);
   A.max_rounds = 16;

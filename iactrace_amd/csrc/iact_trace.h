@@ -94,6 +94,7 @@ struct TraceArgs {
   const float* mirrors;
   int n_surfaces;
   iact_surface surfaces[IACT_MAX_SURFACES];
+  uint32_t conic_surfaces;       // bit i: surface i has no nonzero aspheric term
   iact_obstructions ob;
   DevSensor S;
   // outputs / scratch
@@ -454,7 +455,7 @@ IACT_DEV m3 facet_rotation(const float* rotations, int f) {
 
 // Aperture test of a stage>=1 mirror (mirrors.py:147-149 disk,
 // 209-220 convex CCW polygon).
-IACT_DEV bool in_aperture(const float* M, float x, float y) {
+IACT_DEV bool in_aperture(cptr<float> M, float x, float y) {
   if (M[17] == 0.f) return x * x + y * y <= M[18] * M[18];
   const int n = (int)M[19];
   bool ok = true;
@@ -474,26 +475,36 @@ struct MirrorHit {
   f3 pl, nl;
 };
 
-IACT_DEV MirrorHit mirror_hit(const TraceArgs& A, const float* M, f3 ol, f3 dl) {
-  const iact_surface& su = A.surfaces[(int)M[38]];
-  const SurfT<double> s64 = load_surface<double>(su);
+IACT_DEV MirrorHit mirror_hit(const TraceArgs& A, cptr<float> M, f3 ol, f3 dl) {
+  const int si = (int)M[38];
+  const iact_surface& su = A.surfaces[si];
+  SurfT<double> s64 = load_surface<double>(su);
+  SurfT<float> s32 = load_surface<float>(su);
+  const bool conic = ((A.conic_surfaces >> si) & 1u) != 0u;
+  if (conic) s64.na = s32.na = 0;
   const double x0 = (double)M[15], y0 = (double)M[16];
-  const double z0 = sag_raw<double>(s64, x0, y0);
+  // (both are 0 for a mirror without offset)
+  double z0 = 0.0;
+  float z0f = 0.f;
+  if (M[15] != 0.f || M[16] != 0.f) {
+    z0 = sag_raw<double>(s64, x0, y0);
+    z0f = sag_raw<float>(s32, M[15], M[16]);
+  }
   const double t0 = intersect_conic((double)ol.x + x0, (double)ol.y + y0, (double)ol.z + z0,
-                                    (double)dl.x, (double)dl.y, (double)dl.z, s64.c, s64.k);
+                                    (double)dl.x, (double)dl.y, (double)dl.z, s64.c, s64.k,
+                                    conic && s64.K <= 0.0);
   bool ok;
   const double t = newton_t(s64, ol.x, ol.y, ol.z, dl.x, dl.y, dl.z, x0, y0, z0, t0, ok);
   MirrorHit h;
   const float xh = (float)((double)ol.x + t * (double)dl.x);
   const float yh = (float)((double)ol.y + t * (double)dl.y);
-  const SurfT<float> s32 = load_surface<float>(su);
-  const float z0f = sag_raw<float>(s32, M[15], M[16]);
   surface_point_normal(s32, xh, yh, M[15], M[16], z0f, h.pl, h.nl);
   h.t = (ok && in_aperture(M, xh, yh)) ? (float)t : __builtin_inff();
   return h;
 }
 
-IACT_DEV m3 mirror_rotation(const float* M) {
+template <typename Ptr>
+IACT_DEV m3 mirror_rotation(Ptr M) {
   m3 R;
 #pragma unroll
   for (int i = 0; i < 9; ++i) R.m[i] = M[6 + i];
@@ -523,7 +534,7 @@ IACT_DEV void stage_forward(const TraceArgs& A, int stage, f3& o, f3& d, float& 
   int bi = -1;
   float bx = 0.f, by = 0.f;
   for (int i = 0; i < A.n_mirrors; ++i) {
-    const float* M = A.mirrors + (size_t)IACT_MIRROR_STRIDE * i;
+    const cptr<float> M = as_const(A.mirrors) + (size_t)IACT_MIRROR_STRIDE * i;
     if ((int)M[36] != stage) continue;
     const m3 R = mirror_rotation(M);
     const f3 pos = mk3(M[0], M[1], M[2]);

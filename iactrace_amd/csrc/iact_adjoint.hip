@@ -193,9 +193,12 @@ IACT_DEV void wave_add_keyed(double* table, int key, double v) {
 // frame, so by the implicit function theorem dt = -(m.dol + t m.ddl -
 // dS/da da) / (m.dl) with m = (-Sx, -Sy, 1); the hit point is (x, y, S(x, y))
 // and the normal m / |m|, whose change with (x, y) needs the sag's Hessian.
-// Gradients of the hit surface's aspheric coefficients go to g_asph.
+// Gradients of the hit surface's aspheric coefficients go to g_asph
+// (want_asph): summed per lane in asph_lane where the stage's mirrors share one
+// surface (one_surface), into asph_table otherwise.
 IACT_DEV void stage_adjoint(const AdjArgs& B, const StageRec& rec, f3& go, f3& gr, float& gv,
-                            bool want_asph, double* asph_table) {
+                            bool want_asph, bool one_surface, double* asph_lane,
+                            double* asph_table) {
   const TraceArgs& A = B.T;
   const f3 zero = mk3(0.f, 0.f, 0.f);
   const bool live = rec.mi >= 0 && rec.hs != 0.f;
@@ -242,7 +245,10 @@ IACT_DEV void stage_adjoint(const AdjArgs& B, const StageRec& rec, f3& go, f3& g
       const float dS = pw - pw0;                      // d S / d a_i
       const float dg = (float)(2 * (i + 1)) * D.r2 * q;  // d (dz/dr2) / d a_i
       const float ga = fmaf(gS + k, dS, 2.f * dg * (gSx * D.X + gSy * D.Y));
-      wave_add_keyed(asph_table, use ? IACT_MAX_ASPHERIC * si + i : -1, (double)ga);
+      if (one_surface)
+        asph_lane[i] += use ? (double)ga : 0.0;
+      else
+        wave_add_keyed(asph_table, use ? IACT_MAX_ASPHERIC * si + i : -1, (double)ga);
       pw *= r4;
       pw0 *= r40;
       q *= r4;
@@ -275,14 +281,35 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_adj(AdjArgs B) {
   const bool want_asph = !BATCH && B.g_asph != nullptr && B.surface_index != nullptr &&
                          B.offsets != nullptr;
   const bool want_stage_asph = STAGES && B.g_asph != nullptr;
-  // stage mirrors' aspheric gradients: summed per block in LDS (every wave
-  // of every block adds to the same few coefficients, which as global
-  // atomics serialise) and added to g_asph once per block at the end
-  __shared__ double s_gasph[STAGES ? IACT_MAX_SURFACES * IACT_MAX_ASPHERIC : 1];
-  if (want_stage_asph) {
+  // aspheric gradients: summed per block in LDS (every wave of every block
+  // adds to the same few coefficients, which as global atomics serialise) and
+  // added to g_asph once per block at the end; a stage's own terms per lane
+  // until then
+  __shared__ double s_gasph[BATCH ? 1 : IACT_MAX_SURFACES * IACT_MAX_ASPHERIC];
+  if (want_asph || want_stage_asph) {
     for (int i = threadIdx.x; i < IACT_MAX_SURFACES * IACT_MAX_ASPHERIC; i += blockDim.x)
       s_gasph[i] = 0.0;
     __syncthreads();
+  }
+  // the surface that all mirrors of a stage share, or -1; the lane's sums of
+  // its coefficients' gradients over all rays of the wave
+  int stage_surf[IACT_ADJ_MAX_STAGES];
+  double stage_ga[IACT_ADJ_MAX_STAGES][IACT_MAX_ASPHERIC];
+#pragma unroll
+  for (int k = 0; k < IACT_ADJ_MAX_STAGES; ++k) {
+    stage_surf[k] = -1;
+#pragma unroll
+    for (int i = 0; i < IACT_MAX_ASPHERIC; ++i) stage_ga[k][i] = 0.0;
+    if (!want_stage_asph || k >= A.n_stages) continue;
+    bool one = true;
+    for (int i = 0; i < A.n_mirrors; ++i) {
+      const cptr<float> M = as_const(A.mirrors) + (size_t)IACT_MIRROR_STRIDE * i;
+      if ((int)M[36] != A.stages[k]) continue;
+      const int si = (int)M[38];
+      one = one && (stage_surf[k] < 0 || stage_surf[k] == si);
+      stage_surf[k] = si;
+    }
+    if (!one) stage_surf[k] = -1;
   }
   const long long n_items = total_items(A);
   const long long n_bitems = (n_items + wpb - 1) / wpb;
@@ -329,6 +356,8 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_adj(AdjArgs B) {
     const double* src = A.sources + 3 * w.sbase;
     const cptr<float> vals = as_const(A.values + w.sbase);
     f3 e_lane = mk3(0.f, 0.f, 0.f);  // source offsets, 64 at a time (see k_trace)
+    f3 g_lane = mk3(0.f, 0.f, 0.f);  // source and value gradients, 64 at a time
+    float gval_lane = 0.f;
     long long chunk = -1;            // candidate mask per source chunk (see k_trace)
     for (int si = s0; si < s1; ++si) {
       // the source index as an opaque scalar: derived lane values (s + lane)
@@ -398,7 +427,8 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_adj(AdjArgs B) {
       if (STAGES) {
 #pragma unroll
         for (int k = IACT_ADJ_MAX_STAGES - 1; k >= 0; --k)
-          if (k < A.n_stages) stage_adjoint(B, rec[k], go, gr, gv, want_stage_asph, s_gasph);
+          if (k < A.n_stages) stage_adjoint(B, rec[k], go, gr, gv, want_stage_asph, stage_surf[k] >= 0,
+                                             stage_ga[k], s_gasph);
       }
       // now (go, gr, gv) are the adjoints of the primary leg's origin (the
       // sample), reflected direction and value = value_s * c * nrw * shadow
@@ -443,19 +473,28 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_adj(AdjArgs B) {
         }
       }
       if (want_src || want_val) {
+        // lane k keeps the sums of the k-th source of 64, added to memory
+        // together: the few sources' entries are shared by every wave of the
+        // launch, and an atomic per (wave, source) queued on their cache lines
+        // (382 x 256 x 150 splat rays: 443 us, 267 without the queue)
         const float a = want_src ? wave_sum(active ? gsx : 0.f) : 0.f;
         const float b = want_src ? wave_sum(active ? gsy : 0.f) : 0.f;
         const float cz = want_src ? wave_sum(active ? gsz : 0.f) : 0.f;
         const float e = want_val ? wave_sum(gv * vunit) : 0.f;
-        if (lane == 0) {
+        if (lane == k) {
+          g_lane = mk3(a, b, cz);
+          gval_lane = e;
+        }
+        if ((k == 63 || si + 1 == s1) && lane <= k) {
           // sources the host sorted report to the caller's index
-          const long long so = B.src_perm ? (long long)as_const(B.src_perm)[s] : (long long)s;
+          const int sl = s - k + lane;
+          const long long so = B.src_perm ? (long long)B.src_perm[sl] : (long long)sl;
           if (want_src) {
-            unsafeAtomicAdd(B.g_src + 3 * so, (double)a);
-            unsafeAtomicAdd(B.g_src + 3 * so + 1, (double)b);
-            unsafeAtomicAdd(B.g_src + 3 * so + 2, (double)cz);
+            unsafeAtomicAdd(B.g_src + 3 * so, (double)g_lane.x);
+            unsafeAtomicAdd(B.g_src + 3 * so + 1, (double)g_lane.y);
+            unsafeAtomicAdd(B.g_src + 3 * so + 2, (double)g_lane.z);
           }
-          if (want_val) unsafeAtomicAdd(B.g_val + so, (double)e);
+          if (want_val) unsafeAtomicAdd(B.g_val + so, (double)gval_lane);
         }
       }
     }
@@ -538,7 +577,7 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_adj(AdjArgs B) {
         const float dzx = 2.f * X * dg, dzy = 2.f * Y * dg;  // d (zx, zy) / d a_i
         const float contrib = active ? fmaf(gpl.z, dz, -(gm.x * dzx + gm.y * dzy)) : 0.f;
         const float tot = wave_sum(contrib);
-        if (lane == 0) unsafeAtomicAdd(B.g_asph + IACT_MAX_ASPHERIC * si + i, (double)tot);
+        if (lane == 0) unsafeAtomicAdd(s_gasph + IACT_MAX_ASPHERIC * si + i, (double)tot);
         pw_ *= r4;
         pw0 *= r40;
         q *= r4;
@@ -546,6 +585,18 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_adj(AdjArgs B) {
     }
   }
   if (want_stage_asph) {
+#pragma unroll
+    for (int k = 0; k < IACT_ADJ_MAX_STAGES; ++k) {
+      if (stage_surf[k] < 0) continue;
+#pragma unroll
+      for (int i = 0; i < IACT_MAX_ASPHERIC; ++i) {
+        if (i >= A.surfaces[stage_surf[k]].n_aspheric) break;
+        const double v = wave_sum_d(stage_ga[k][i]);
+        if (lane == 0) unsafeAtomicAdd(s_gasph + IACT_MAX_ASPHERIC * stage_surf[k] + i, v);
+      }
+    }
+  }
+  if (want_asph || want_stage_asph) {
     __syncthreads();
     for (int i = threadIdx.x; i < IACT_MAX_SURFACES * IACT_MAX_ASPHERIC; i += blockDim.x) {
       const double v = s_gasph[i];

@@ -379,6 +379,17 @@ int shape_trace(const iact_scene& sc, int ns, int mode, const iact_launch* L, Tr
   if (mode == IACT_MODE_IMAGE && !A.det && sc.n_stages == 0 && sm_fits &&
       (lay == 2 || (lay == 0 && ns >= 64)))
     A.layout = 2;
+  // Images and response rows in fp64 where they fit (see lds_add): 592 against
+  // 184 us for 382 x 256 x 150 rays of seven splat taps.  A hard source-major
+  // image has an add per run of rays and keeps the smaller entries.  Rays of
+  // further stages are scattered enough to be added as they are (8192 x 2048
+  // rays: 827 us with 16 merging rounds, 656 with none); the rays of one facet
+  // and source are merged once, as all 64 may meet one pixel.
+  if (A.lds_image && !A.det && (A.layout != 2 || A.S.splat) && 2 * img + tab <= budget) {
+    A.lds_image = 2;
+    A.max_rounds = sc.n_stages > 0 ? 0 : 1;
+    out.lds += img;
+  }
   // obstruction culling
   A.cull = nullptr;
   int rc = cull_words_for(sc, L, A.cull_words, A.cull_all);
@@ -392,12 +403,20 @@ int shape_trace(const iact_scene& sc, int ns, int mode, const iact_launch* L, Tr
     long long sg = (L && L->sample_group) ? L->sample_group : 64;
     if (sg < 1) return set_error(IACT_ERR_INVALID, "sample_group %lld", sg);
     // two sources per lane from 128 sources: a sample's record, loop control
-    // and facet bookkeeping then serve two rays per lane
-    A.sm_spl = ns >= 128 ? 2 : 1;
+    // and facet bookkeeping then serve two rays per lane (a splat ray's taps
+    // outweigh both)
+    A.sm_spl = ns >= 128 && !A.S.splat ? 2 : 1;
     const long long cw = 64ll * A.sm_spl;
     const long long n_sc = ns > 0 ? (ns + cw - 1) / cw : 1;
     // items are decoded in 32 bits
     while (((total + sg - 1) / sg) * n_sc >= (1ll << 31)) sg *= 2;
+    if (A.S.splat && !(L && L->sample_group)) {
+      // a splat item of 64 samples takes some 30 us: smaller ones until each
+      // wave of the smallest grid has eight, or the last ones decide (382 x 256
+      // samples x 150 sources, whole call: 273 us in items of 64, 195 of 16, 187 of 8)
+      const long long want = 8ll * 4 * dev.n_cu * wpb;
+      while (sg > 8 && ((total + sg - 1) / sg) * n_sc < want) sg /= 2;
+    }
     if (sg > total) sg = total > 0 ? total : 1;
     A.sample_group = (int)sg;
     A.n_sc = (uint32_t)n_sc;

@@ -74,11 +74,14 @@ IACT_DEV void plane_adjoint(const DevSensor& S, f3 r, float t, float gx, float g
 }
 
 // Splat tap weights and their gradient w.r.t. the sensor-plane hit:
-// returns sum_k G_k w_k and writes dL/dx, dL/dy for a ray of value v.
-template <int KIND>
-IACT_DEV float splat_adjoint(const DevSensor& S, const int32_t* table, const float* G, float x,
-                             float y, bool ok_in, float v, float& gx, float& gy) {
-  const int ks = S.ks;
+// returns sum_k G_k w_k and writes dL/dx, dL/dy for a ray of value v.  KS: as
+// in splat_taps_ks.
+template <int KIND, int KS>
+IACT_DEV float splat_adjoint_ks(const DevSensor& S, const int32_t* table, const float* G, float x,
+                                float y, bool ok_in, float v, float& gx, float& gy) {
+  const int ks = KS ? KS : S.ks;
+  constexpr int D = 2 * KS + 1;
+  float ew[D * D];
   const float h2 = 2.f * S.neg_half_inv_sigma2;
   gx = 0.f;
   gy = 0.f;
@@ -87,10 +90,13 @@ IACT_DEV float splat_adjoint(const DevSensor& S, const int32_t* table, const flo
     const float xb = floorf(xp), yb = floorf(yp);
     const float xf = xp - xb, yf = yp - yb;
     float tot = 0.f, sx = 0.f, sy = 0.f;
+#pragma unroll
     for (int oy = -ks; oy <= ks; ++oy)
+#pragma unroll
       for (int ox = -ks; ox <= ks; ++ox) {
         const float ex = xf - (float)ox, ey = yf - (float)oy;
         const float e = __expf(S.neg_half_inv_sigma2 * fmaf(ex, ex, ey * ey));
+        if (KS) ew[(oy + KS) * D + ox + KS] = e;
         tot += e;
         sx = fmaf(e, ex, sx);
         sy = fmaf(e, ey, sy);
@@ -100,13 +106,17 @@ IACT_DEV float splat_adjoint(const DevSensor& S, const int32_t* table, const flo
     const float it = frcp(tot);
     const float mx = sx * it, my = sy * it;
     float gw = 0.f, ax = 0.f, ay = 0.f;
+#pragma unroll
     for (int oy = -ks; oy <= ks; ++oy)
+#pragma unroll
       for (int ox = -ks; ox <= ks; ++ox) {
         const float ex = xf - (float)ox, ey = yf - (float)oy;
-        const float w = __expf(S.neg_half_inv_sigma2 * fmaf(ex, ex, ey * ey)) * it;
+        const float w = (KS ? ew[(oy + KS) * D + ox + KS]
+                            : __expf(S.neg_half_inv_sigma2 * fmaf(ex, ex, ey * ey))) *
+                        it;
         const float xi = xb + (float)ox, yi = yb + (float)oy;
         const bool in = xi >= 0.f && xi < S.wf && yi >= 0.f && yi < S.hf;
-        const float g = in ? G[(int)yi * S.width + (int)xi] : 0.f;
+        const float g = in ? G[(int)fmaf(yi, S.wf, xi)] : 0.f;
         gw = fmaf(g, w, gw);
         ax = fmaf(g * w, ex - mx, ax);
         ay = fmaf(g * w, ey - my, ay);
@@ -119,52 +129,66 @@ IACT_DEV float splat_adjoint(const DevSensor& S, const int32_t* table, const flo
     hex_axial(S, x, y, q, r);
     hex_round(q, r, qb, rb);
     const float dq = q - qb, dr = r - rb;
+    // a tap's hex norm and h2 hd_k (d hd_k / d(dq, dr)) = d ln e_k / d(dq, dr)
+    auto tap = [&](int oq, int orr, float& hd, float& tq, float& tr) {
+      const float a0 = dq - (float)oq, b0 = dr - (float)orr;
+      hd = hex_norm_axial(a0, b0);
+      const float ee = fmaf(0.5f, b0, a0);
+      const float se = ee > 0.f ? 1.f : (ee < 0.f ? -1.f : 0.f);
+      const float sb = b0 > 0.f ? 1.f : (b0 < 0.f ? -1.f : 0.f);
+      const bool first = 2.f * fabsf(ee) >= fmaf(1.5f, fabsf(b0), fabsf(ee));
+      tq = h2 * hd * (first ? 2.f * se : se);
+      tr = h2 * hd * (first ? se : fmaf(0.5f, se, 1.5f * sb));
+    };
     float tot = 0.f, sq = 0.f, sr = 0.f;
-    // d ln e_k / d(dq, dr) = h2 hd_k (d hd_k / d(dq, dr))
+#pragma unroll
     for (int oq = -ks; oq <= ks; ++oq)
+#pragma unroll
       for (int orr = -ks; orr <= ks; ++orr) {
-        if (max(max(abs(oq), abs(orr)), abs(oq + orr)) > ks) continue;
-        const float a0 = dq - (float)oq, b0 = dr - (float)orr;
-        const float hd = hex_norm_axial(a0, b0);
+        if (!hex_tap(oq, orr, ks)) continue;
+        float hd, tq, tr;
+        tap(oq, orr, hd, tq, tr);
         const float e = __expf(S.neg_half_inv_sigma2 * hd * hd);
-        const float ee = fmaf(0.5f, b0, a0);
-        const float se = ee > 0.f ? 1.f : (ee < 0.f ? -1.f : 0.f);
-        const float sb = b0 > 0.f ? 1.f : (b0 < 0.f ? -1.f : 0.f);
-        const bool first = 2.f * fabsf(ee) >= fmaf(1.5f, fabsf(b0), fabsf(ee));
-        const float da = first ? 2.f * se : se;
-        const float db = first ? se : fmaf(0.5f, se, 1.5f * sb);
+        if (KS) ew[(oq + KS) * D + orr + KS] = e;
         tot += e;
-        sq = fmaf(e, h2 * hd * da, sq);
-        sr = fmaf(e, h2 * hd * db, sr);
+        sq = fmaf(e, tq, sq);
+        sr = fmaf(e, tr, sr);
       }
     const bool ok = ok_in && tot > 0.f && fabsf(qb) < 1e8f && fabsf(rb) < 1e8f;
     if (!ok) return 0.f;
     const float it = frcp(tot);
     const float mq = sq * it, mr = sr * it;
+    const HexTaps<KS> T(S, qb, rb);
     float gw = 0.f, aq = 0.f, ar = 0.f;
+#pragma unroll
     for (int oq = -ks; oq <= ks; ++oq)
+#pragma unroll
       for (int orr = -ks; orr <= ks; ++orr) {
-        if (max(max(abs(oq), abs(orr)), abs(oq + orr)) > ks) continue;
-        const float a0 = dq - (float)oq, b0 = dr - (float)orr;
-        const float hd = hex_norm_axial(a0, b0);
-        const float w = __expf(S.neg_half_inv_sigma2 * hd * hd) * it;
-        const float ee = fmaf(0.5f, b0, a0);
-        const float se = ee > 0.f ? 1.f : (ee < 0.f ? -1.f : 0.f);
-        const float sb = b0 > 0.f ? 1.f : (b0 < 0.f ? -1.f : 0.f);
-        const bool first = 2.f * fabsf(ee) >= fmaf(1.5f, fabsf(b0), fabsf(ee));
-        const float da = first ? 2.f * se : se;
-        const float db = first ? se : fmaf(0.5f, se, 1.5f * sb);
-        const int pid = hex_lookup(S, table, qb + (float)oq, rb + (float)orr);
+        if (!hex_tap(oq, orr, ks)) continue;
+        float hd, tq, tr;
+        tap(oq, orr, hd, tq, tr);
+        const float w = (KS ? ew[(oq + KS) * D + orr + KS]
+                            : __expf(S.neg_half_inv_sigma2 * hd * hd)) *
+                        it;
+        const int pid = KS ? T.at(S, table, oq, orr)
+                           : hex_lookup(S, table, qb + (float)oq, rb + (float)orr);
         const float g = pid >= 0 ? G[pid] : 0.f;
         gw = fmaf(g, w, gw);
-        aq = fmaf(g * w, h2 * hd * da - mq, aq);
-        ar = fmaf(g * w, h2 * hd * db - mr, ar);
+        aq = fmaf(g * w, tq - mq, aq);
+        ar = fmaf(g * w, tr - mr, ar);
       }
     const float gq = v * aq, gr = v * ar;
     gx = fmaf(gq, S.aqx, gr * S.arx);
     gy = fmaf(gq, S.aqy, gr * S.ary);
     return gw;
   }
+}
+template <int KIND>
+IACT_DEV float splat_adjoint(const DevSensor& S, const int32_t* table, const float* G, float x,
+                             float y, bool ok, float v, float& gx, float& gy) {
+  if (S.ks == 1) return splat_adjoint_ks<KIND, 1>(S, table, G, x, y, ok, v, gx, gy);
+  if (S.ks == 2) return splat_adjoint_ks<KIND, 2>(S, table, G, x, y, ok, v, gx, gy);
+  return splat_adjoint_ks<KIND, 0>(S, table, G, x, y, ok, v, gx, gy);
 }
 
 // Stages >= 1 whose reflections the adjoint follows (the host rejects more).

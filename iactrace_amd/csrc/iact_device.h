@@ -948,23 +948,18 @@ IACT_DEV double wave_sum_d(double v) {
   return v;
 }
 
-// Add every lane's value into img[pix] (pix < 0: nothing).  Lanes that share
-// a pixel are summed across the wave first so the LDS (or global) image sees
-// one atomic per distinct pixel; after `max_rounds` distinct pixels the rest
-// add directly.  Must be called by the whole wave in uniform control flow.
-template <bool GLOBAL, class T>
-IACT_DEV void wave_accumulate(T* img, int pix, float v, int max_rounds) {
+// Give every lane's value to add(pix, v) (pix < 0: nothing).  Lanes that share
+// a pixel are summed across the wave first so the image sees one add per
+// distinct pixel; after `max_rounds` distinct pixels the rest add directly.
+// Must be called by the whole wave in uniform control flow.
+template <typename Add>
+IACT_DEV void wave_accumulate(int pix, float v, int max_rounds, Add&& add) {
   uint64_t rem = __ballot(pix >= 0 && v != 0.f);
   int rounds = 0;
   const int lane = lane_id();
   while (rem) {
     if (rounds == max_rounds) {
-      if ((rem >> lane) & 1ull) {
-        if (GLOBAL)
-          unsafeAtomicAdd(img + pix, (T)v);
-        else
-          atomicAdd(img + pix, (T)v);
-      }
+      if ((rem >> lane) & 1ull) add(pix, v);
       break;
     }
     const int leader = __builtin_ctzll(rem);
@@ -972,15 +967,32 @@ IACT_DEV void wave_accumulate(T* img, int pix, float v, int max_rounds) {
     const bool mine = ((rem >> lane) & 1ull) && pix == key;
     const uint64_t m = __ballot(mine);
     const float s = wave_sum(mine ? v : 0.f);
-    if (lane == leader) {
-      if (GLOBAL)
-        unsafeAtomicAdd(img + key, (T)s);
-      else
-        atomicAdd(img + key, (T)s);
-    }
+    if (lane == leader) add(key, s);
     rem &= ~m;
     ++rounds;
   }
 }
+
+// A block's image in LDS, fp32 or fp64 entries (uniform over the launch).
+struct LdsImage {
+  float* f;
+  double* d;
+  bool f64;
+  IACT_DEV void add(int pix, float v) const {
+    if (f64)
+      lds_add(d + pix, v);
+    else
+      lds_add(f + pix, v);
+  }
+  IACT_DEV void clear(int n) const {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+      if (f64)
+        d[i] = 0.0;
+      else
+        f[i] = 0.f;
+    }
+  }
+  IACT_DEV double at(int i) const { return f64 ? d[i] : (double)f[i]; }
+};
 
 }  // namespace iact

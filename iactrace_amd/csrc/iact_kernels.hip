@@ -357,13 +357,16 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_accumulate(DevSensor S, cons
     if (!SPLAT) {
       const int pix = active ? hard_pixel<KIND>(S, tab, xi, yi) : -1;
       if (pixel && active) pixel[i] = pix;
-      wave_accumulate<true>(out, pix, vi, 16);
+      wave_accumulate(pix, vi, 16, [&](int p, float a) { unsafeAtomicAdd(out + p, a); });
     } else {
       if (pixel && active) pixel[i] = hard_pixel<KIND>(S, tab, xi, yi);
       float gu, gv;
       to_grid<KIND>(S, xi, yi, gu, gv);
       splat_taps<KIND>(S, tab, gu, gv, active,
-                       [&](int pix, float w) { wave_accumulate<true>(out, pix, vi * w, 16); });
+                       [&](int pix, float w) {
+                         wave_accumulate(pix, vi * w, 16,
+                                         [&](int p, float a) { unsafeAtomicAdd(out + p, a); });
+                       });
     }
   }
 }
@@ -406,17 +409,17 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace(TraceArgs A) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wpb = block_waves();
   const int lane = lane_id();
   const int P = A.S.n_pixels;
-  float* img_lds = smem;
-  int32_t* tab_lds = (int32_t*)(smem + (lds_image ? (det ? wpb : 1) * P : 0));
-  if (MODE == IACT_MODE_IMAGE && lds_image) {
-    const int n = (det ? wpb : 1) * P;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) img_lds[i] = 0.f;
-  }
+  const bool f64 = A.lds_image == 2;
+  const int n_img = (det ? wpb : 1) * P;
+  const LdsImage block_img{smem, (double*)smem, f64};
+  int32_t* tab_lds = (int32_t*)(smem + (lds_image ? n_img << (f64 ? 1 : 0) : 0));
+  if (MODE == IACT_MODE_IMAGE && lds_image) block_img.clear(n_img);
   // hex tables are always staged in LDS
   const int32_t* table =
       KIND == IACT_SENSOR_HEX && A.lds_table ? stage_hex_table(A.S, tab_lds) : tab_lds;
   __syncthreads();
-  float* img = img_lds + (det ? wave * P : 0);
+  // (deterministic: the wave's own image, fp32)
+  const LdsImage img{smem + (det ? wave * P : 0), (double*)smem, f64};
 
   int run_pix = -1;
   float run_v = 0.f;
@@ -430,10 +433,10 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace(TraceArgs A) {
     if (MODE == IACT_MODE_IMAGE && lds_image && inst != cur) {
       __syncthreads();
       for (int i = threadIdx.x; i < P; i += blockDim.x) {
-        const float v = img_lds[i];
-        if (v != 0.f) unsafeAtomicAdd(A.out64 + (size_t)cur * P + i, (double)v);
-        img_lds[i] = 0.f;
+        const double v = block_img.at(i);
+        if (v != 0.0) unsafeAtomicAdd(A.out64 + (size_t)cur * P + i, v);
       }
+      block_img.clear(P);
       __syncthreads();
     }
     cur = inst;
@@ -453,6 +456,8 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace(TraceArgs A) {
     Sample smp = make_sample<KIND>(A.S, pw, nw, A.weights[gi], pos);
     const int s0 = w.s0, s1 = w.s1;
     double* const gout = A.out64 + (size_t)w.inst * P;
+    const auto to_lds = [&](int p, float a) { img.add(p, a); };
+    const auto to_mem = [&](int p, float a) { unsafeAtomicAdd(gout + p, (double)a); };
     const double* src = A.sources + 3 * w.sbase;
     const cptr<float> vals = as_const(A.values + w.sbase);
     // the facet's source offsets, 64 sources at a time (lane k holds source
@@ -491,42 +496,42 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace(TraceArgs A) {
         if (lds_image && acc == 1) {
           // per-lane run of equal pixels, flushed when the pixel changes
           if (pix != run_pix) {
-            if (run_pix >= 0 && run_v != 0.f) atomicAdd(img + run_pix, run_v);
+            if (run_pix >= 0 && run_v != 0.f) img.add(run_pix, run_v);
             run_pix = pix;
             run_v = 0.f;
           }
           run_v += v;  // a run of pix = -1 is never added
         } else if (lds_image && acc == 2) {
-          if (pix >= 0 && v != 0.f) atomicAdd(img + pix, v);
+          if (pix >= 0 && v != 0.f) img.add(pix, v);
         } else if (lds_image) {
-          wave_accumulate<false>(img, pix, v, A.max_rounds);
+          wave_accumulate(pix, v, A.max_rounds, to_lds);
         } else {
-          wave_accumulate<true>(gout, pix, v, A.max_rounds);
+          wave_accumulate(pix, v, A.max_rounds, to_mem);
         }
       } else {
         splat_taps<KIND>(A.S, table, gu, gv, ok, [&](int pix, float wt) {
           if (lds_image)
-            wave_accumulate<false>(img, pix, v * wt, A.max_rounds);
+            wave_accumulate(pix, v * wt, A.max_rounds, to_lds);
           else
-            wave_accumulate<true>(gout, pix, v * wt, A.max_rounds);
+            wave_accumulate(pix, v * wt, A.max_rounds, to_mem);
         });
       }
     }
   }
 
   if (MODE == IACT_MODE_IMAGE && lds_image) {
-    if (!SPLAT && acc == 1 && run_pix >= 0 && run_v != 0.f) atomicAdd(img + run_pix, run_v);
+    if (!SPLAT && acc == 1 && run_pix >= 0 && run_v != 0.f) img.add(run_pix, run_v);
     __syncthreads();
     if (det) {
       for (int i = threadIdx.x; i < P; i += blockDim.x) {
         float s = 0.f;
-        for (int w = 0; w < wpb; ++w) s += img_lds[w * P + i];
+        for (int w = 0; w < wpb; ++w) s += smem[w * P + i];
         A.partials[(size_t)blockIdx.x * P + i] = s;
       }
     } else {
       for (int i = threadIdx.x; i < P; i += blockDim.x) {
-        const float v = img_lds[i];
-        if (v != 0.f) unsafeAtomicAdd(A.out64 + (size_t)cur * P + i, (double)v);
+        const double v = block_img.at(i);
+        if (v != 0.0) unsafeAtomicAdd(A.out64 + (size_t)cur * P + i, v);
       }
     }
   }
@@ -662,7 +667,7 @@ IACT_DEV bool refine_candidates(const TraceArgs& A, int f, int c, int blk, int l
 // each with its own register allocation), and it is 5 % faster than at 5
 // waves and 8 % faster than at 7, whose register limit moves spills into the
 // per-ray loop.
-template <int SRC, int KIND, int SPLAT, bool STAGES, bool AXIS, int OBST, int SPL>
+template <int SRC, int KIND, int SPLAT, int OBST, int SPL>
 __global__ __launch_bounds__(IACT_MAX_BLOCK)
 __attribute__((amdgpu_waves_per_eu(OBST ? 6 : 1))) void k_trace_sm(TraceArgs A) {
   extern __shared__ float smem[];
@@ -671,10 +676,10 @@ __attribute__((amdgpu_waves_per_eu(OBST ? 6 : 1))) void k_trace_sm(TraceArgs A) 
   const int P = A.S.n_pixels;
   // the LDS image behind one spare entry, img[-1]: a run of pixel -1 (no
   // pixel yet, or dropped rays) is added there, without a test
-  float* img = smem + 1;
-  int32_t* tab_lds = (int32_t*)(smem + (A.lds_image ? P + 1 : 0));
-  if (A.lds_image)
-    for (int i = threadIdx.x; i < P; i += blockDim.x) img[i] = 0.f;
+  const bool f64 = SPLAT && A.lds_image == 2;
+  const LdsImage img{smem + 1, (double*)smem + 1, f64};
+  int32_t* tab_lds = (int32_t*)(smem + (A.lds_image ? (P + 1) << (f64 ? 1 : 0) : 0));
+  if (A.lds_image) img.clear(P);
   const int32_t* table =
       KIND == IACT_SENSOR_HEX && A.lds_table ? stage_hex_table(A.S, tab_lds) : tab_lds;
   __syncthreads();
@@ -684,7 +689,7 @@ __attribute__((amdgpu_waves_per_eu(OBST ? 6 : 1))) void k_trace_sm(TraceArgs A) 
   // make it a flat atomic, which also stalls the record prefetch)
   auto add_run = [&](int pix, float v) {
     if (A.lds_image)
-      lds_add(img + pix, v);
+      img.add(pix, v);
     else if (pix >= 0 && v != 0.f)
       unsafeAtomicAdd(A.out64 + pix, (double)v);
   };
@@ -760,7 +765,7 @@ __attribute__((amdgpu_waves_per_eu(OBST ? 6 : 1))) void k_trace_sm(TraceArgs A) 
         float gu, gv, v, x, y, vf, cu;
         // a ray's value is linear in its source's: hard binning traces unit
         // values and scales a run once, when it is added
-        const bool ok = trace_ray<SRC, KIND, STAGES, AXIS, OB, false, GEN, FR>(
+        const bool ok = trace_ray<SRC, KIND, false, false, OB, false, GEN, FR>(
             A, smp, true, e[k], qs[k], SPLAT ? value[k] : 1.f, gu, gv, v, x, y, &vf, &cu);
         if (SB) {
           // the run's shadow bits (far_run_shadow) in place of the test
@@ -780,10 +785,9 @@ __attribute__((amdgpu_waves_per_eu(OBST ? 6 : 1))) void k_trace_sm(TraceArgs A) 
             run_v[k] = 0.f;
             run_l[k] = 0.f;
           }
-          // a run of pix = -1 is never added; without shadow tests and
-          // stages v = vf * nrwh, summed in one fma (far runs: v = cu nrwh
-          // run_s)
-          if (OB || STAGES)
+          // a run of pix = -1 is never added; without shadow tests
+          // v = vf * nrwh, summed in one fma (far runs: v = cu nrwh run_s)
+          if (OB)
             run_v[k] += v;
           else if (SRC == IACT_SOURCE_POINT && FR)
             run_l[k] = fmaf(cu, smp.nrwh, run_l[k]);
@@ -903,8 +907,8 @@ __attribute__((amdgpu_waves_per_eu(OBST ? 6 : 1))) void k_trace_sm(TraceArgs A) 
   if (A.lds_image) {
     __syncthreads();
     for (int i = threadIdx.x; i < P; i += blockDim.x) {
-      const float v = img[i];
-      if (v != 0.f) unsafeAtomicAdd(A.out64 + i, (double)v);
+      const double v = img.at(i);
+      if (v != 0.0) unsafeAtomicAdd(A.out64 + i, v);
     }
   }
 }
@@ -935,7 +939,7 @@ __attribute__((amdgpu_waves_per_eu(OBST ? 6 : 1))) void k_trace_sm(TraceArgs A) 
 // and 3 % faster than the rotation-only kernel at 5 waves without spills.
 // GX false: the launch wants rotation gradients only (no value, source or
 // position gradients), and the kernel has no code or registers for the rest.
-template <int SRC, int KIND, bool AXIS, int OBST, int SPL, bool GX>
+template <int SRC, int KIND, int OBST, int SPL, bool GX>
 __global__ __launch_bounds__(IACT_MAX_BLOCK)
 __attribute__((amdgpu_waves_per_eu(6))) void k_adj_sm(AdjArgs B) {
   const TraceArgs& A = B.T;
@@ -1245,8 +1249,8 @@ template <int SRC, int KIND, int SPLAT>
 __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_response(TraceArgs A) {
   extern __shared__ float smem[];
   const int P = A.S.n_pixels;
-  float* row = smem;
-  int32_t* tab_lds = (int32_t*)(smem + (A.lds_image ? P : 0));
+  const LdsImage row{smem, (double*)smem, A.lds_image == 2};
+  int32_t* tab_lds = (int32_t*)(smem + (A.lds_image ? P << (row.f64 ? 1 : 0) : 0));
   const int32_t* table =
       KIND == IACT_SENSOR_HEX && A.lds_table ? stage_hex_table(A.S, tab_lds) : tab_lds;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wpb = block_waves();
@@ -1254,10 +1258,11 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_response(TraceArgs A) 
   const long long total = (long long)A.nf * A.M;
   const long long nchunks = (long long)A.nf * A.cpf;
   for (int s = blockIdx.x; s < A.ns; s += grid_blocks()) {
-    if (A.lds_image)
-      for (int i = threadIdx.x; i < P; i += blockDim.x) row[i] = 0.f;
+    if (A.lds_image) row.clear(P);
     __syncthreads();
     float* gdst = A.out + (size_t)s * P;
+    const auto to_lds = [&](int p, float a) { row.add(p, a); };
+    const auto to_mem = [&](int p, float a) { unsafeAtomicAdd(gdst + p, a); };
     const double sx = A.sources[3 * s], sy = A.sources[3 * s + 1], sz = A.sources[3 * s + 2];
     const float val = A.values[s];
     int fe = -1;
@@ -1284,21 +1289,21 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_response(TraceArgs A) 
       if (!SPLAT) {
         const int pix = grid_pixel<KIND>(A.S, table, gu, gv, ok);
         if (A.lds_image)
-          wave_accumulate<false>(row, pix, v, A.max_rounds);
+          wave_accumulate(pix, v, A.max_rounds, to_lds);
         else
-          wave_accumulate<true>(gdst, pix, v, A.max_rounds);
+          wave_accumulate(pix, v, A.max_rounds, to_mem);
       } else {
         splat_taps<KIND>(A.S, table, gu, gv, ok, [&](int pix, float w) {
           if (A.lds_image)
-            wave_accumulate<false>(row, pix, v * w, A.max_rounds);
+            wave_accumulate(pix, v * w, A.max_rounds, to_lds);
           else
-            wave_accumulate<true>(gdst, pix, v * w, A.max_rounds);
+            wave_accumulate(pix, v * w, A.max_rounds, to_mem);
         });
       }
     }
     __syncthreads();
     if (A.lds_image)
-      for (int i = threadIdx.x; i < P; i += blockDim.x) A.out[(size_t)s * P + i] = row[i];
+      for (int i = threadIdx.x; i < P; i += blockDim.x) gdst[i] = (float)row.at(i);
     __syncthreads();
   }
 }
@@ -1357,18 +1362,13 @@ static TraceKernel pick_trace_t(const TraceArgs& A) {
 
 // source-major kernels exist for primary-only scenes (the host selects that
 // layout only for those); obstructed scenes take the kernel with the shadow
-// path
-template <int SRC, int KIND, int SPLAT, int SPL>
-static TraceKernel pick_sm_spl(const TraceArgs& A) {
-  if (has_obstructions(A.ob))
-    return A.S.axis ? k_trace_sm<SRC, KIND, SPLAT, false, true, 1, SPL>
-                    : k_trace_sm<SRC, KIND, SPLAT, false, false, 1, SPL>;
-  return A.S.axis ? k_trace_sm<SRC, KIND, SPLAT, false, true, 0, SPL>
-                  : k_trace_sm<SRC, KIND, SPLAT, false, false, 0, SPL>;
-}
+// path; splat kernels have one source per lane (see shape_trace)
 template <int SRC, int KIND, int SPLAT>
 static TraceKernel pick_sm_t(const TraceArgs& A) {
-  return A.sm_spl == 2 ? pick_sm_spl<SRC, KIND, SPLAT, 2>(A) : pick_sm_spl<SRC, KIND, SPLAT, 1>(A);
+  const bool ob = has_obstructions(A.ob);
+  if (!SPLAT && A.sm_spl == 2)
+    return ob ? k_trace_sm<SRC, KIND, 0, 1, 2> : k_trace_sm<SRC, KIND, 0, 0, 2>;
+  return ob ? k_trace_sm<SRC, KIND, SPLAT, 1, 1> : k_trace_sm<SRC, KIND, SPLAT, 0, 1>;
 }
 
 template <int SRC>
@@ -1423,21 +1423,18 @@ hipError_t launch_trace_sm(const TraceArgs& A, const LaunchShape& L, int source_
   return launch_trace_kernel(pick_trace_kernel(A, source_type, TRACE_SOURCE_MAJOR), A, L, st);
 }
 
-template <int SRC, int KIND, bool AXIS, int SPL>
+template <int SRC, int KIND, int SPL>
 static const void* pick_adj_sm_spl(const AdjArgs& B) {
-  const bool gx = B.g_val || B.g_src || B.g_pos;
+  const bool gx = B.g_src || B.g_val || B.g_pos;
   if (has_obstructions(B.T.ob))
-    return gx ? (const void*)k_adj_sm<SRC, KIND, AXIS, 1, SPL, true>
-              : (const void*)k_adj_sm<SRC, KIND, AXIS, 1, SPL, false>;
-  return gx ? (const void*)k_adj_sm<SRC, KIND, AXIS, 0, SPL, true>
-            : (const void*)k_adj_sm<SRC, KIND, AXIS, 0, SPL, false>;
+    return gx ? (const void*)k_adj_sm<SRC, KIND, 1, SPL, true>
+              : (const void*)k_adj_sm<SRC, KIND, 1, SPL, false>;
+  return gx ? (const void*)k_adj_sm<SRC, KIND, 0, SPL, true>
+            : (const void*)k_adj_sm<SRC, KIND, 0, SPL, false>;
 }
 template <int SRC, int KIND>
 static const void* pick_adj_sm_k(const AdjArgs& B) {
-  const bool ax = B.T.S.axis != 0;
-  if (B.T.sm_spl == 2)
-    return ax ? pick_adj_sm_spl<SRC, KIND, true, 2>(B) : pick_adj_sm_spl<SRC, KIND, false, 2>(B);
-  return ax ? pick_adj_sm_spl<SRC, KIND, true, 1>(B) : pick_adj_sm_spl<SRC, KIND, false, 1>(B);
+  return B.T.sm_spl == 2 ? pick_adj_sm_spl<SRC, KIND, 2>(B) : pick_adj_sm_spl<SRC, KIND, 1>(B);
 }
 template <int SRC>
 static const void* pick_adj_sm(const AdjArgs& B) {

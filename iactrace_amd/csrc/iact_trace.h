@@ -108,10 +108,10 @@ struct TraceArgs {
   int32_t* dbg_pix;
   float* partials;
   const float* world;  // SoA (7, nf*M) when precomputed
-  int lds_image;       // image accumulated in LDS: 1 fp32, 2 fp64 (source-major)
+  int lds_image;       // image accumulated in LDS: 1 fp32, 2 fp64
   int lds_table;       // hex table staged in LDS
   int det;             // deterministic (wave-private images, ordered sums)
-  int max_rounds;
+  int max_rounds;      // of wave_accumulate
   int acc;             // 0 wave-merged, 1 per-lane run-length, 2 direct atomics
   // work order (see decode_item)
   uint32_t span;       // chunks per block of the order
@@ -921,30 +921,64 @@ IACT_DEV void to_grid(const DevSensor& S, float x, float y, float& gu, float& gv
   }
 }
 
+// Pixel ids of the splat taps around the cell (qb, rb) from the bordered table:
+// clamped rows and columns read the border's -1, so one clamp per row and
+// column serves all taps.
+template <int KS>
+struct HexTaps {
+  int row[2 * KS + 1], col[2 * KS + 1];
+  IACT_DEV HexTaps(const DevSensor& S, float qb, float rb) {
+#pragma unroll
+    for (int i = 0; i <= 2 * KS; ++i) {
+      row[i] = floor_i32(__builtin_amdgcn_fmed3f(qb + (float)(i - KS + 1), 0.f, S.tq_f + 1.f));
+      col[i] = floor_i32(__builtin_amdgcn_fmed3f(rb + (float)(i - KS + 1), 0.f, S.tr_f + 1.f));
+    }
+  }
+  IACT_DEV int at(const DevSensor& S, const int32_t* table, int oq, int orr) const {
+    return table[__umul24((unsigned)row[oq + KS], (unsigned)(S.tr + 2)) + (unsigned)col[orr + KS]];
+  }
+};
+IACT_DEV constexpr bool hex_tap(int oq, int orr, int ks) {
+  const int s = oq + orr;
+  return oq <= ks && -oq <= ks && orr <= ks && -orr <= ks && s <= ks && -s <= ks;
+}
+
 // Splat taps of one ray (square.py:144-173, hexagonal.py:264-315).  Calls
 // fn(pixel, weight) for every tap; weights are normalised to sum 1.  Rays
 // that miss the plane or whose normaliser underflows contribute nothing.
-// The hit is given in sensor-grid coordinates (gu, gv).
-template <int KIND, typename Fn>
-IACT_DEV void splat_taps(const DevSensor& S, const int32_t* table, float gu, float gv,
-                         bool ok_in, Fn&& fn) {
-  const int ks = S.ks;
+// The hit is given in sensor-grid coordinates (gu, gv).  KS: the kernel size
+// (1, 2) when it is known -- the loops then unroll and every tap's exponential
+// is formed once -- or 0.
+template <int KIND, int KS, typename Fn>
+IACT_DEV void splat_taps_ks(const DevSensor& S, const int32_t* table, float gu, float gv,
+                            bool ok_in, Fn&& fn) {
+  const int ks = KS ? KS : S.ks;
+  constexpr int D = 2 * KS + 1;
+  float ew[D * D];
   if (KIND == IACT_SENSOR_SQUARE) {
     const float xp = gu, yp = gv;
     const float xb = floorf(xp), yb = floorf(yp);
     const float xf = xp - xb, yf = yp - yb;
+    auto tap = [&](int oy, int ox) {
+      const float ex = xf - (float)ox, ey = yf - (float)oy;
+      return __expf(S.neg_half_inv_sigma2 * fmaf(ex, ex, ey * ey));
+    };
     float tot = 0.f;
+#pragma unroll
     for (int oy = -ks; oy <= ks; ++oy)
+#pragma unroll
       for (int ox = -ks; ox <= ks; ++ox) {
-        const float ex = xf - (float)ox, ey = yf - (float)oy;
-        tot += __expf(S.neg_half_inv_sigma2 * fmaf(ex, ex, ey * ey));
+        const float e = tap(oy, ox);
+        if (KS) ew[(oy + KS) * D + ox + KS] = e;
+        tot += e;
       }
     const bool ok = ok_in && tot > 0.f && fabsf(xb) < 1e8f && fabsf(yb) < 1e8f;
     const float it = ok ? frcp(tot) : 0.f;
+#pragma unroll
     for (int oy = -ks; oy <= ks; ++oy)
+#pragma unroll
       for (int ox = -ks; ox <= ks; ++ox) {
-        const float ex = xf - (float)ox, ey = yf - (float)oy;
-        const float w = __expf(S.neg_half_inv_sigma2 * fmaf(ex, ex, ey * ey)) * it;
+        const float w = (KS ? ew[(oy + KS) * D + ox + KS] : tap(oy, ox)) * it;
         const float xi = xb + (float)ox, yi = yb + (float)oy;
         const bool in = ok && xi >= 0.f && xi < S.wf && yi >= 0.f && yi < S.hf;
         fn(in ? (int)fmaf(yi, S.wf, xi) : -1, w);
@@ -954,24 +988,45 @@ IACT_DEV void splat_taps(const DevSensor& S, const int32_t* table, float gu, flo
     float qb, rb;
     hex_round(q, r, qb, rb);
     const float dq = q - qb, dr = r - rb;
+    auto tap = [&](int oq, int orr) {
+      const float hd = hex_norm_axial(dq - (float)oq, dr - (float)orr);
+      return __expf(S.neg_half_inv_sigma2 * hd * hd);
+    };
     float tot = 0.f;
+#pragma unroll
     for (int oq = -ks; oq <= ks; ++oq)
+#pragma unroll
       for (int orr = -ks; orr <= ks; ++orr) {
-        if (max(max(abs(oq), abs(orr)), abs(oq + orr)) > ks) continue;
-        const float hd = hex_norm_axial(dq - (float)oq, dr - (float)orr);
-        tot += __expf(S.neg_half_inv_sigma2 * hd * hd);
+        if (!hex_tap(oq, orr, ks)) continue;
+        const float e = tap(oq, orr);
+        if (KS) ew[(oq + KS) * D + orr + KS] = e;
+        tot += e;
       }
     const bool ok = ok_in && tot > 0.f && fabsf(qb) < 1e8f && fabsf(rb) < 1e8f;
     const float it = ok ? frcp(tot) : 0.f;
+    const HexTaps<KS> T(S, qb, rb);
+#pragma unroll
     for (int oq = -ks; oq <= ks; ++oq)
+#pragma unroll
       for (int orr = -ks; orr <= ks; ++orr) {
-        if (max(max(abs(oq), abs(orr)), abs(oq + orr)) > ks) continue;
-        const float hd = hex_norm_axial(dq - (float)oq, dr - (float)orr);
-        const float w = __expf(S.neg_half_inv_sigma2 * hd * hd) * it;
-        const int pid = ok ? hex_lookup(S, table, qb + (float)oq, rb + (float)orr) : -1;
+        if (!hex_tap(oq, orr, ks)) continue;
+        const float w = (KS ? ew[(oq + KS) * D + orr + KS] : tap(oq, orr)) * it;
+        const int pid = !ok ? -1
+                        : KS ? T.at(S, table, oq, orr)
+                             : hex_lookup(S, table, qb + (float)oq, rb + (float)orr);
         fn(pid, w);
       }
   }
+}
+template <int KIND, typename Fn>
+IACT_DEV void splat_taps(const DevSensor& S, const int32_t* table, float gu, float gv,
+                         bool ok_in, Fn&& fn) {
+  if (S.ks == 1)
+    splat_taps_ks<KIND, 1>(S, table, gu, gv, ok_in, fn);
+  else if (S.ks == 2)
+    splat_taps_ks<KIND, 2>(S, table, gu, gv, ok_in, fn);
+  else
+    splat_taps_ks<KIND, 0>(S, table, gu, gv, ok_in, fn);
 }
 
 }  // namespace iact

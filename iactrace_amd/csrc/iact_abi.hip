@@ -304,6 +304,21 @@ int work_order(const iact_launch* L, long long nchunks, int grid, int wpb, Trace
   return IACT_OK;
 }
 
+// Tile and parts of k_response: two sources per block where LDS has room, and
+// parts of at least two chunks per wave until there are eight blocks per CU.
+// 382 x 64 samples x 4096 sources, 960 hexagons, masts, whole call with tiles of
+// 1, 2, 4: 521, 419, 439 us; 875 x 256 x 300, 2048 hexagons: 456, 331, 357.
+static void shape_response(TraceArgs& A, int ns, long long nchunks, size_t row, size_t tab,
+                           const DevInfo& dev) {
+  A.resp_tile = 2 * row + tab <= 65536 ? 2 : 1;
+  const long long tiles = (ns + A.resp_tile - 1) / A.resp_tile;
+  const long long most = nchunks / (2 * (IACT_RESPONSE_BLOCK / 64));
+  long long parts = (8ll * dev.n_cu + tiles - 1) / tiles;
+  if (parts > most) parts = most;
+  A.resp_parts = parts > 1 ? (int)parts : 1;
+  A.d_parts = make_fastdiv((uint32_t)A.resp_parts);
+}
+
 int shape_trace(const iact_scene& sc, int ns, int mode, const iact_launch* L, TraceArgs& A,
                 LaunchShape& out, const DevInfo& dev, int source_type) {
   const int threads = (L && L->block_threads) ? L->block_threads : 256;
@@ -390,6 +405,9 @@ int shape_trace(const iact_scene& sc, int ns, int mode, const iact_launch* L, Tr
     A.max_rounds = sc.n_stages > 0 ? 0 : 1;
     out.lds += img;
   }
+  if (mode == IACT_MODE_RESPONSE && !A.det && sc.n_stages == 0 && !A.S.splat && sm_fits &&
+      A.lds_image == 2 && ns > 0 && nch > 0 && nch < (1ll << 31))
+    shape_response(A, ns, nch, (size_t)P * sizeof(double), tab, dev);
   // obstruction culling
   A.cull = nullptr;
   int rc = cull_words_for(sc, L, A.cull_words, A.cull_all);
@@ -465,9 +483,9 @@ int regrid(long long items, const iact_launch* L, const DevInfo& dev, LaunchShap
 
 static size_t base_workspace_bytes(const iact_scene& sc, int mode, const LaunchShape& shp,
                                    const TraceArgs& A) {
-  if (mode == IACT_MODE_RESPONSE)
+  if (mode == IACT_MODE_RESPONSE && !A.resp_tile)
     return (size_t)7 * sc.facets.n_facets * sc.facets.n_samples * sizeof(float);
-  if (mode == IACT_MODE_IMAGE && A.layout == 2)
+  if (mode == IACT_MODE_RESPONSE || (mode == IACT_MODE_IMAGE && A.layout == 2))
     // two records of padding: the trace prefetches up to two records ahead
     return (size_t)IACT_REC_WORDS * ((size_t)sc.facets.n_facets * sc.facets.n_samples + 2) *
            sizeof(float);
@@ -739,6 +757,7 @@ static size_t workspace_size(const iact_scene* scene, int32_t n_sources, int32_t
   fill_trace_args(A, *scene, nullptr, nullptr, n_sources);
   LaunchShape shp;
   if (shape_trace(*scene, n_sources, mode, launch, A, shp, dev, -1)) return 0;
+  if (!tree) A.resp_tile = 0;
   return workspace_bytes_for(*scene, n_sources, mode, shp, A, dev, tree);
 }
 
@@ -778,6 +797,7 @@ static int32_t trace_fwd(const iact_scene* scene, const double* sources, const f
   LaunchShape shp;
   rc = shape_trace(sc, n_sources, mode, launch, A, shp, dev, source_type);
   if (rc) return rc;
+  if (!want_tree) A.resp_tile = 0;
   const size_t need = workspace_bytes_for(sc, n_sources, mode, shp, A, dev, want_tree);
   if (need > 0 && (!workspace || workspace_bytes < need))
     return set_error(IACT_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need,
@@ -844,11 +864,18 @@ static int32_t trace_fwd(const iact_scene* scene, const double* sources, const f
     return IACT_OK;
   }
   if (mode == IACT_MODE_RESPONSE) {
-    if (n_sources > 0 && (empty || !A.lds_image)) {
+    if (n_sources > 0 && (empty || !A.lds_image || (A.resp_tile && A.resp_parts > 1))) {
       e = launch_fill(out, (long long)n_sources * P, 0.f, st);
       if (e != hipSuccess) return hip_error(e, "clear response matrix");
     }
     if (empty) return IACT_OK;
+    if (A.resp_tile) {
+      A.recs = (const float*)workspace;
+      e = launch_records(A, (float*)workspace, st);
+      if (e != hipSuccess) return hip_error(e, "k_sample_records");
+      e = launch_response(A, source_type, st);
+      return e == hipSuccess ? IACT_OK : hip_error(e, "k_response");
+    }
     float* world = (float*)workspace;
     e = launch_world(sc.facets, A.S, world, st);
     if (e != hipSuccess) return hip_error(e, "k_facet_world");

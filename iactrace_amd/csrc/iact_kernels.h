@@ -4,6 +4,7 @@
 #include "iact_trace.h"
 
 #define IACT_MAX_BLOCK 256
+#define IACT_RESPONSE_BLOCK 512  // threads of k_response
 
 namespace iact {
 
@@ -32,6 +33,9 @@ hipError_t launch_accumulate(const DevSensor& S, const float* x, const float* y,
                              long long n, float* out, int32_t* pixel, hipStream_t st);
 hipError_t launch_trace_sm(const TraceArgs& A, const LaunchShape& L, int source_type,
                            hipStream_t st);
+// Response matrix of a primary-only, hard-binned scene (A.resp_tile > 0) from
+// the sample records.
+hipError_t launch_response(const TraceArgs& A, int source_type, hipStream_t st);
 hipError_t launch_records(const TraceArgs& A, float* recs, hipStream_t st);
 hipError_t launch_cull(const TraceArgs& A, int source_type, int all, float* cones,
                        uint32_t* masks, hipStream_t st);

@@ -1308,6 +1308,75 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_response(TraceArgs A) 
   }
 }
 
+// Response matrix of a primary-only, hard-binned scene: a block owns resp_tile
+// sources (fp64 rows in LDS) and a part of the sample chunks; a lane's sample
+// record is loaded once for the tile's sources.  Within a facet the records are
+// sorted by aperture position.  Blocks of one part write their rows whole; with
+// several parts (few sources, which would leave CUs idle) they add what they
+// have to rows cleared before.  VALU issue bounds it, and where a facet's rays
+// meet one pixel the LDS adds, which is why lanes are merged once before.
+// 382 x 64 samples x 4096 sources behind masts: 805 us with one source per block
+// and samples prepared per ray, 373 now; 382 x 256 samples x 64 sources: 454 -> 75 us
+// for the whole call.
+template <int SRC, int KIND, int OBST>
+__global__ __launch_bounds__(IACT_RESPONSE_BLOCK) void k_response(TraceArgs A) {
+  extern __shared__ double rows[];
+  const int P = A.S.n_pixels, T = A.resp_tile;
+  const int tile = (int)fdiv(blockIdx.x, A.d_parts), part = blockIdx.x - tile * A.resp_parts;
+  const int s0 = tile * T, n_src = min(T, A.ns - s0);
+  for (int i = threadIdx.x; i < n_src * P; i += IACT_RESPONSE_BLOCK) rows[i] = 0.0;
+  int32_t* tab_lds = (int32_t*)(rows + T * P);
+  const int32_t* table = KIND == IACT_SENSOR_HEX ? stage_hex_table(A.S, tab_lds) : tab_lds;
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
+  const long long total = (long long)A.nf * A.M;
+  const bool lean = as_const((const uint32_t*)(A.recs + IACT_REC_WORDS * total))[0] == 0u &&
+                    !A.S.edge && (KIND != IACT_SENSOR_SQUARE || A.S.v_scale == 1.f);
+  const long long nchunks = (long long)A.nf * A.cpf;
+  const int c0 = (int)(nchunks * part / A.resp_parts);
+  const int c1 = (int)(nchunks * (part + 1) / A.resp_parts);
+  const double* sp = A.sources + 3 * (size_t)(s0 + min(lane, n_src - 1));
+  const double sx = sp[0], sy = sp[1], sz = sp[2];
+  const cptr<float> vals = as_const(A.values) + s0;
+  for (int c = c0 + wave; c < c1; c += IACT_RESPONSE_BLOCK / 64) {
+    const int f = (int)fdiv((uint32_t)c, A.d_cpf);
+    const int m = (c - f * A.cpf) * 64 + lane;
+    const bool active = m < A.M;
+    const float4* rp = (const float4*)A.recs + 4 * ((size_t)f * A.M + (active ? m : A.M - 1));
+    Sample smp = unpack_record(RecRaw{rp[0], rp[1], rp[2], rp[3]});
+    const FacetCull fc = OBST ? facet_cull(A, f, s0 >> 6) : FacetCull{f, 0u, 0, 0};
+    set_facet(smp, fc);
+    const cptr<float> fp = as_const(A.positions) + 3 * f;
+    const f3 e_lane = source_offset<SRC>(sx, sy, sz, mk3(fp[0], fp[1], fp[2]));
+    auto trace = [&](auto sh, auto gen) {
+      constexpr bool GEN = decltype(gen)::value;
+      for (int k = 0; k < n_src; ++k) {
+        const f3 e = lane_value(e_lane, k);
+        float gu, gv, v, x, y;
+        const bool ok = trace_ray<SRC, KIND, false, false, decltype(sh)::value ? 1 : 0, false, GEN>(
+            A, smp, active, e, source_qs(A, e), vals[k], gu, gv, v, x, y);
+        const int pix = grid_pixel<KIND, GEN>(A.S, table, gu, gv, ok);
+        wave_accumulate(pix, v, A.max_rounds, [&](int p, float a) { lds_add(rows + k * P + p, a); });
+      }
+    };
+    if (OBST && fc.any)
+      trace(std::true_type{}, std::true_type{});
+    else if (lean)
+      trace(std::false_type{}, std::false_type{});
+    else
+      trace(std::false_type{}, std::true_type{});
+  }
+  __syncthreads();
+  float* const out = A.out + (size_t)s0 * P;
+  for (int i = threadIdx.x; i < n_src * P; i += IACT_RESPONSE_BLOCK) {
+    const double v = rows[i];
+    if (A.resp_parts == 1)
+      out[i] = (float)v;
+    else if (v != 0.0)
+      unsafeAtomicAdd(out + i, (float)v);
+  }
+}
+
 // ------------------------------------------------------------------ launchers
 static int grid_for(long long n, int threads, int cap) {
   long long g = (n + threads - 1) / threads;
@@ -1421,6 +1490,25 @@ hipError_t launch_trace(const TraceArgs& A, const LaunchShape& L, int source_typ
 hipError_t launch_trace_sm(const TraceArgs& A, const LaunchShape& L, int source_type,
                            hipStream_t st) {
   return launch_trace_kernel(pick_trace_kernel(A, source_type, TRACE_SOURCE_MAJOR), A, L, st);
+}
+
+template <int SRC>
+static TraceKernel pick_response(const TraceArgs& A) {
+  const bool ob = has_obstructions(A.ob);
+  if (A.S.kind == IACT_SENSOR_SQUARE)
+    return ob ? k_response<SRC, IACT_SENSOR_SQUARE, 1> : k_response<SRC, IACT_SENSOR_SQUARE, 0>;
+  return ob ? k_response<SRC, IACT_SENSOR_HEX, 1> : k_response<SRC, IACT_SENSOR_HEX, 0>;
+}
+hipError_t launch_response(const TraceArgs& A, int source_type, hipStream_t st) {
+  const size_t tab = A.S.kind == IACT_SENSOR_HEX
+                         ? (size_t)(A.S.tq + 2) * (A.S.tr + 2) * sizeof(int32_t)
+                         : 0;
+  const LaunchShape L{((A.ns + A.resp_tile - 1) / A.resp_tile) * A.resp_parts, 0,
+                      IACT_RESPONSE_BLOCK,
+                      (size_t)A.resp_tile * A.S.n_pixels * sizeof(double) + tab};
+  return launch_trace_kernel(source_type == IACT_SOURCE_POINT ? pick_response<IACT_SOURCE_POINT>(A)
+                                                              : pick_response<IACT_SOURCE_PARALLEL>(A),
+                             A, L, st);
 }
 
 template <int SRC, int KIND, int SPL>

@@ -108,6 +108,10 @@ struct TraceArgs {
   int32_t* dbg_pix;
   float* partials;
   const float* world;  // SoA (7, nf*M) when precomputed
+  // response matrix from sample records (k_response): sources per block (0: not
+  // taken), parts of the sample chunks
+  int resp_tile, resp_parts;
+  FastDiv d_parts;
   int lds_image;       // image accumulated in LDS: 1 fp32, 2 fp64
   int lds_table;       // hex table staged in LDS
   int det;             // deterministic (wave-private images, ordered sums)

@@ -77,6 +77,8 @@ def _stages(groups):
 
 
 def _f32c(t, device):
+    if t.dtype is torch.float32 and t.device == device and t.is_contiguous():
+        return t  # (read through its address only)
     return t.detach().to(device=device, dtype=torch.float32).contiguous()
 
 
@@ -103,8 +105,17 @@ def sample_radius(points):
     return r
 
 
-def facets_abi(groups, keep, rotations=None, positions=None):
-    """IactFacets over the concatenation of stage-0 ``groups`` (render.py:201-205)."""
+def _surface_index(groups, device):
+    """Each facet's group, on the device."""
+    idx = torch.cat([torch.full((len(g),), i, dtype=torch.int32) for i, g in enumerate(groups)])
+    return idx.to(device)
+
+
+def facets_abi(groups, keep, rotations=None, positions=None, surface_index=None):
+    """IactFacets over the concatenation of stage-0 ``groups`` (render.py:201-205).
+    surface_index: _surface_index of the groups where the caller holds it (made
+    here, it is a copy from host memory, which waits for the stream: 16 us of a
+    60 us call on one star, and no call could be prepared while one ran)."""
     dev = groups[0].positions.device
     F = _lib.IactFacets()
     F.n_facets = sum(len(g) for g in groups)
@@ -127,8 +138,7 @@ def facets_abi(groups, keep, rotations=None, positions=None):
     # the far-source test of the kernels bounds every sample's offset from
     # its facet position by this radius
     F.max_sample_radius = max(sample_radius(g.points) for g in groups)
-    sidx = torch.cat([torch.full((len(g),), i, dtype=torch.int32) for i, g in enumerate(groups)])
-    arrs["surface_index"] = sidx.to(dev)
+    arrs["surface_index"] = _surface_index(groups, dev) if surface_index is None else surface_index
     for k, v in arrs.items():
         keep.append(v)
         setattr(F, k, v.data_ptr())
@@ -214,14 +224,13 @@ class RenderPlan:
         ob = pack_obstruction_tables(self.tel.obstruction_groups or [])
         self.obstruction_tables = {k: torch.as_tensor(v).to(dev).contiguous() for k, v in ob.items()}
         self.sensor_abi = self.sensor.to_abi(dev)
+        self.surface_index = _surface_index(self.primary, dev) if self.primary else None
+        self.static_scene = self._static_scene()
 
-    def scene(self, keep, rotations=None, positions=None):
+    def _static_scene(self):
+        """Scene descriptor without its facets and surfaces."""
         sc = _lib.IactScene()
-        if self.primary:
-            sc.facets = facets_abi(self.primary, keep, rotations, positions)
         sc.n_surfaces = len(self.surface_groups)
-        for i, g in enumerate(self.surface_groups):
-            sc.surfaces[i] = g.surface_abi()
         sc.n_mirrors = self.mirror_table.shape[0]
         sc.mirrors = self.mirror_table.data_ptr() if sc.n_mirrors else None
         sc.n_stages = len(self.stages)
@@ -238,6 +247,14 @@ class RenderPlan:
             setattr(o, cnt, t.shape[0])
             setattr(o, field, t.data_ptr() if t.shape[0] else None)
         sc.sensor = self.sensor_abi
+        return sc
+
+    def scene(self, keep, rotations=None, positions=None):
+        sc = _lib.IactScene.from_buffer_copy(self.static_scene)
+        if self.primary:
+            sc.facets = facets_abi(self.primary, keep, rotations, positions, self.surface_index)
+        for i, g in enumerate(self.surface_groups):
+            sc.surfaces[i] = g.surface_abi()
         return sc
 
     # ------------------------------------------------------------ forward
@@ -349,9 +366,11 @@ class _TraceFunction(torch.autograd.Function):
         g_rot = _like(outs["rotations"], rotations) if nig[4] else None
         g_pos = _like(outs["positions"], positions) if nig[5] else None
         g_asph = []
-        for i in range(ctx.n_asph):
+        asph = [ctx.plan.surface_groups[i].aspheric for i in range(ctx.n_asph)]
+        if need[4] and all(a.device.type == "cpu" for a in asph):
+            outs["aspheric"] = outs["aspheric"].cpu()  # (one wait for all of them)
+        for i, a in enumerate(asph):
             if nig[6 + i]:
-                a = ctx.plan.surface_groups[i].aspheric
                 g = outs["aspheric"][i, :a.numel()].to(device=a.device, dtype=a.dtype)
                 g_asph.append(g.reshape(a.shape))
             else:

@@ -640,6 +640,15 @@ int adj_sm_layout(const iact_scene& sc, const double* sources, const float* valu
 
 long long refine_groups(const TraceArgs& A, int mode) {
   if (mode != IACT_MODE_IMAGE || A.layout != 2 || !has_obstructions(A.ob)) return 0;
+bool tree_shared(const iact_scene& sc, int ns, const iact_launch* L, const DevInfo& dev) {
+  if (sc.facets.n_facets <= 0 || ns <= 0 || !bwd_source_major(sc, ns, L, false)) return false;
+  TraceArgs A;
+  fill_trace_args(A, sc, nullptr, nullptr, ns);
+  LaunchShape shp, ts;
+  if (shape_trace(sc, ns, IACT_MODE_IMAGE, L, A, shp, dev, -1)) return false;
+  return tree_serves(A, 0, 0, dev, ts) && tree_serves(A, 1, 0, dev, ts);
+}
+
   return ((long long)A.nf * A.M + 63) / 64;
 }
 
@@ -814,7 +823,7 @@ static int32_t trace_fwd(const iact_scene* scene, const double* sources, const f
     memset(&B, 0, sizeof(B));
     B.T = A;
     B.T.partials = (float*)((char*)workspace + T.sums);
-    return launch_tree(B, T, workspace, tshp, source_type, 0, 0, st);
+    return launch_tree(B, T, workspace, tshp, source_type, 0, 0, false, st);
   }
   if (!empty) {
     const CullSpec c{n_sources, 1, nullptr, mode == IACT_MODE_IMAGE && !A.det,

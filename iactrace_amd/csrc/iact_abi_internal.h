@@ -74,7 +74,15 @@ int tree_max_grid(const DevInfo& dev);
 // 2 keeps per source (1 value gradients, 4 also source gradients, else 0).
 bool tree_serves(const TraceArgs& A, int mode, int n_acc, const DevInfo& dev, LaunchShape& shp);
 int launch_tree(AdjArgs& B, const TreeLayout& T, void* workspace, const LaunchShape& shp,
-                int source_type, int mode, int n_acc, hipStream_t st);
+                int source_type, int mode, int n_acc, bool built, hipStream_t st);
+// Whether an image launch and a rotation gradient of it both walk the tree, whose
+// preparation the second can then take over from the first; and that gradient
+// (iact_trace_bwd with tree_built).
+bool tree_shared(const iact_scene& sc, int ns, const iact_launch* L, const DevInfo& dev);
+int trace_bwd(const iact_scene* scene, const double* sources, const float* values,
+              int32_t n_sources, int32_t source_type, const float* grad_image,
+              const iact_launch* launch, void* workspace, size_t workspace_bytes,
+              const iact_grads* grads, bool tree_built, void* stream);
 // An image or gradient launch may reorder its sources into direction cells.
 inline bool tree_sorts(const TraceArgs& A, int ns) {
   return A.cull_words > 0 && !A.cull_all && ns >= kChunkCullMinSources;

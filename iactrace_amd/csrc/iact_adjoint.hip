@@ -668,38 +668,10 @@ hipError_t launch_adjoint(const AdjArgs& B, const LaunchShape& L, int source_typ
                          args, L.lds, st);
 }
 
-}  // namespace iact
-
-using namespace iact;
-
-extern "C" {
-
-size_t iact_bwd_workspace_size(const iact_scene* scene, int32_t n_sources,
-                               const iact_launch* launch) {
-  if (validate_scene(scene) || n_sources < 0) return 0;
-  DevInfo dev;
-  if (device_info(dev)) return 0;
-  TraceArgs A;
-  fill_trace_args(A, *scene, nullptr, nullptr, n_sources);
-  LaunchShape shp;
-  if (shape_trace(*scene, n_sources, IACT_MODE_DEBUG, launch, A, shp, dev, -1)) return 0;
-  const CullSpec c{n_sources, 1, nullptr, true};
-  size_t need = cull_layout(A.nf, A.cull_words, A.cull_all, 0, c).end;
-  // (the source-major adjoint is not taken when aspheric gradients are
-  // requested; the size covers both)
-  if (bwd_source_major(*scene, n_sources, launch, false)) {
-    TraceArgs B;
-    AdjSmLayout lay;
-    if (adj_sm_layout(*scene, nullptr, nullptr, n_sources, launch, dev, B, shp, lay)) return 0;
-    if (lay.end > need) need = lay.end;
-  }
-  return need;
-}
-
-int32_t iact_trace_bwd(const iact_scene* scene, const double* sources, const float* values,
-                       int32_t n_sources, int32_t source_type, const float* grad_image,
-                       const iact_launch* launch, void* workspace, size_t workspace_bytes,
-                       const iact_grads* grads, void* stream) {
+int trace_bwd(const iact_scene* scene, const double* sources, const float* values,
+              int32_t n_sources, int32_t source_type, const float* grad_image,
+              const iact_launch* launch, void* workspace, size_t workspace_bytes,
+              const iact_grads* grads, bool tree_built, void* stream) {
   int rc = validate_scene(scene);
   if (rc) return rc;
   if (!grads) return set_error(IACT_ERR_INVALID, "null gradient descriptor");
@@ -759,7 +731,7 @@ int32_t iact_trace_bwd(const iact_scene* scene, const double* sources, const flo
       B.torque = (double*)((char*)workspace + T.sums);
       e = launch_fill_d(B.torque, 3ll * nf, 0.0, st);
       if (e != hipSuccess) return hip_error(e, "clear torques");
-      rc = launch_tree(B, T, workspace, tshp, source_type, mode, n_acc, st);
+      rc = launch_tree(B, T, workspace, tshp, source_type, mode, n_acc, tree_built, st);
       if (rc) return rc;
       if (grads->rotations) {
         e = launch_torque_to_euler(B.torque, sc.facets.rotations, nf, grads->rotations, st);
@@ -824,6 +796,42 @@ int32_t iact_trace_bwd(const iact_scene* scene, const double* sources, const flo
   if (rc) return rc;
   e = launch_adjoint(B, shp, source_type, st);
   return e == hipSuccess ? IACT_OK : hip_error(e, "k_trace_adj");
+}
+
+}  // namespace iact
+
+using namespace iact;
+
+extern "C" {
+
+size_t iact_bwd_workspace_size(const iact_scene* scene, int32_t n_sources,
+                               const iact_launch* launch) {
+  if (validate_scene(scene) || n_sources < 0) return 0;
+  DevInfo dev;
+  if (device_info(dev)) return 0;
+  TraceArgs A;
+  fill_trace_args(A, *scene, nullptr, nullptr, n_sources);
+  LaunchShape shp;
+  if (shape_trace(*scene, n_sources, IACT_MODE_DEBUG, launch, A, shp, dev, -1)) return 0;
+  const CullSpec c{n_sources, 1, nullptr, true};
+  size_t need = cull_layout(A.nf, A.cull_words, A.cull_all, 0, c).end;
+  // (the source-major adjoint is not taken when aspheric gradients are
+  // requested; the size covers both)
+  if (bwd_source_major(*scene, n_sources, launch, false)) {
+    TraceArgs B;
+    AdjSmLayout lay;
+    if (adj_sm_layout(*scene, nullptr, nullptr, n_sources, launch, dev, B, shp, lay)) return 0;
+    if (lay.end > need) need = lay.end;
+  }
+  return need;
+}
+
+int32_t iact_trace_bwd(const iact_scene* scene, const double* sources, const float* values,
+                       int32_t n_sources, int32_t source_type, const float* grad_image,
+                       const iact_launch* launch, void* workspace, size_t workspace_bytes,
+                       const iact_grads* grads, void* stream) {
+  return trace_bwd(scene, sources, values, n_sources, source_type, grad_image, launch, workspace,
+                   workspace_bytes, grads, false, stream);
 }
 
 }  // extern "C"

@@ -1448,9 +1448,11 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
 }
 
 // The image from the blocks' partial images, summed in fp64: one block per 64
-// pixels, a wave per sixteenth of the partials.
-__global__ __launch_bounds__(1024) void k_sum_partials(const float* part, int n, int P,
-                                                       float* out) {
+// pixels, a wave per sixteenth of the partials.  Leaves the walk's work counter
+// cleared for a gradient walk of the same tree.
+__global__ __launch_bounds__(1024) void k_sum_partials(const float* part, int n, int P, float* out,
+                                                       uint32_t* work) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *work = 0u;
   __shared__ double red[16][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int i = blockIdx.x * 64 + lane;
@@ -1618,42 +1620,48 @@ static const void* pick_tree(const TraceArgs& A, int mode) {
 }
 
 // The whole trace: sorted sources in obstructed scenes (an item's sources then
-// bound a narrow bundle), frame, records, nodes, walk.
+// bound a narrow bundle), frame, records, nodes, walk.  built: an image launch
+// of the same scene, sources and stream has just left all of it but the walk in
+// the workspace.
 int launch_tree(AdjArgs& B, const TreeLayout& T, void* workspace, const LaunchShape& shp,
-                int source_type, int mode, int n_acc, hipStream_t st) {
+                int source_type, int mode, int n_acc, bool built, hipStream_t st) {
   TraceArgs& A = B.T;
   char* ws = (char*)workspace;
   TreeParams K = tree_args(A, T, workspace, shp.full_grid);
   K.n_acc = n_acc;
   hipError_t e;
+  const bool hex = A.S.kind == IACT_SENSOR_HEX;
   if (T.sort) {
     int32_t* pm = (int32_t*)(ws + T.perm);
     double* so = (double*)(ws + T.src);
     float* vo = (float*)(ws + T.val);
-    e = launch_sort_sources(A.sources, A.values, A.ns, nullptr, 1, source_type, ws + T.sws, pm,
-                            so, vo, st);
-    if (e != hipSuccess) return hip_error(e, "source sort");
+    if (!built) {
+      e = launch_sort_sources(A.sources, A.values, A.ns, nullptr, 1, source_type, ws + T.sws, pm,
+                              so, vo, st);
+      if (e != hipSuccess) return hip_error(e, "source sort");
+    }
     A.sources = so;
     A.values = vo;
     B.src_perm = pm;
   }
-  e = launch_records(A, (float*)workspace, st);
-  if (e != hipSuccess) return hip_error(e, "k_sample_records");
-  const int tw = table_words(A.S);
-  hipLaunchKernelGGL(k_tree_frame, dim3(1 + (tw + 1023) / 1024), dim3(1024), 0, st, A.sources,
-                     A.ns, source_type, A.S, (float*)(ws + T.frame), (int16_t*)(ws + T.table));
-  e = hipGetLastError();
-  if (e != hipSuccess) return hip_error(e, "k_tree_frame");
-  const bool hex = A.S.kind == IACT_SENSOR_HEX;
-  const dim3 ng(A.nf * T.n_top);
-  if (hex)
-    hipLaunchKernelGGL(k_tree_nodes<IACT_SENSOR_HEX>, ng, dim3(256), 0, st, A, K,
-                       (float*)(ws + T.nodes), (float*)(ws + T.balls));
-  else
-    hipLaunchKernelGGL(k_tree_nodes<IACT_SENSOR_SQUARE>, ng, dim3(256), 0, st, A, K,
-                       (float*)(ws + T.nodes), (float*)(ws + T.balls));
-  e = hipGetLastError();
-  if (e != hipSuccess) return hip_error(e, "k_tree_nodes");
+  if (!built) {
+    e = launch_records(A, (float*)workspace, st);
+    if (e != hipSuccess) return hip_error(e, "k_sample_records");
+    const int tw = table_words(A.S);
+    hipLaunchKernelGGL(k_tree_frame, dim3(1 + (tw + 1023) / 1024), dim3(1024), 0, st, A.sources,
+                       A.ns, source_type, A.S, (float*)(ws + T.frame), (int16_t*)(ws + T.table));
+    e = hipGetLastError();
+    if (e != hipSuccess) return hip_error(e, "k_tree_frame");
+    const dim3 ng(A.nf * T.n_top);
+    if (hex)
+      hipLaunchKernelGGL(k_tree_nodes<IACT_SENSOR_HEX>, ng, dim3(256), 0, st, A, K,
+                         (float*)(ws + T.nodes), (float*)(ws + T.balls));
+    else
+      hipLaunchKernelGGL(k_tree_nodes<IACT_SENSOR_SQUARE>, ng, dim3(256), 0, st, A, K,
+                         (float*)(ws + T.nodes), (float*)(ws + T.balls));
+    e = hipGetLastError();
+    if (e != hipSuccess) return hip_error(e, "k_tree_nodes");
+  }
   const void* k =
       source_type == IACT_SOURCE_POINT
           ? (hex ? pick_tree<IACT_SOURCE_POINT, IACT_SENSOR_HEX>(A, mode)
@@ -1667,7 +1675,7 @@ int launch_tree(AdjArgs& B, const TreeLayout& T, void* workspace, const LaunchSh
   if (e != hipSuccess) return hip_error(e, "k_tree");
   if (mode == 0) {
     hipLaunchKernelGGL(k_sum_partials, dim3((A.S.n_pixels + 63) / 64), dim3(1024), 0, st,
-                       A.partials, grid, A.S.n_pixels, A.out);
+                       A.partials, grid, A.S.n_pixels, A.out, (uint32_t*)(ws + T.frame) + 4);
     e = hipGetLastError();
     if (e != hipSuccess) return hip_error(e, "k_sum_partials");
   }

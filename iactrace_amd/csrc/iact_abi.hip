@@ -394,15 +394,17 @@ int shape_trace(const iact_scene& sc, int ns, int mode, const iact_launch* L, Tr
   if (mode == IACT_MODE_IMAGE && !A.det && sc.n_stages == 0 && sm_fits &&
       (lay == 2 || (lay == 0 && ns >= 64)))
     A.layout = 2;
-  // Images and response rows in fp64 where they fit (see lds_add): 592 against
-  // 184 us for 382 x 256 x 150 rays of seven splat taps.  A hard source-major
-  // image has an add per run of rays and keeps the smaller entries.  Rays of
-  // further stages are scattered enough to be added as they are (8192 x 2048
-  // rays: 827 us with 16 merging rounds, 656 with none); the rays of one facet
-  // and source are merged once, as all 64 may meet one pixel.
-  if (A.lds_image && !A.det && (A.layout != 2 || A.S.splat) && 2 * img + tab <= budget) {
+  // Splat images, images through further stages and response rows in fp64 where
+  // they fit (see lds_add): 592 against 184 us for 382 x 256 x 150 rays of seven
+  // splat taps.  Rays of further stages are scattered enough to be added as they
+  // are (8192 x 2048 rays: 827 us with 16 merging rounds, 656 with none); the
+  // rays of one facet and source are merged first, as all 64 may meet one pixel.
+  // A hard primary-only image has an add per run of rays or per few merged lanes
+  // and keeps fp32 (875 x 4096 x 40 rays behind masts: 817 us, 862 in fp64).
+  if (A.lds_image && !A.det &&
+      (mode == IACT_MODE_RESPONSE || A.S.splat || sc.n_stages > 0) && 2 * img + tab <= budget) {
     A.lds_image = 2;
-    A.max_rounds = sc.n_stages > 0 ? 0 : 1;
+    A.max_rounds = sc.n_stages > 0 ? 0 : mode == IACT_MODE_RESPONSE ? 1 : 2;
     out.lds += img;
   }
   if (mode == IACT_MODE_RESPONSE && !A.det && sc.n_stages == 0 && !A.S.splat && sm_fits &&
@@ -638,8 +640,6 @@ int adj_sm_layout(const iact_scene& sc, const double* sources, const float* valu
   return IACT_OK;
 }
 
-long long refine_groups(const TraceArgs& A, int mode) {
-  if (mode != IACT_MODE_IMAGE || A.layout != 2 || !has_obstructions(A.ob)) return 0;
 bool tree_shared(const iact_scene& sc, int ns, const iact_launch* L, const DevInfo& dev) {
   if (sc.facets.n_facets <= 0 || ns <= 0 || !bwd_source_major(sc, ns, L, false)) return false;
   TraceArgs A;
@@ -649,6 +649,8 @@ bool tree_shared(const iact_scene& sc, int ns, const iact_launch* L, const DevIn
   return tree_serves(A, 0, 0, dev, ts) && tree_serves(A, 1, 0, dev, ts);
 }
 
+long long refine_groups(const TraceArgs& A, int mode) {
+  if (mode != IACT_MODE_IMAGE || A.layout != 2 || !has_obstructions(A.ob)) return 0;
   return ((long long)A.nf * A.M + 63) / 64;
 }
 

@@ -415,7 +415,7 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_adj(AdjArgs B) {
       if (STAGES) {
 #pragma unroll
         for (int k = 0; k < IACT_ADJ_MAX_STAGES; ++k)
-          if (k < A.n_stages) stage_forward<true>(A, A.stages[k], of, rf, vf, active, rec[k]);
+          if (k < A.n_stages) stage_forward<true, 2>(A, A.stages[k], of, rf, vf, active, rec[k]);
         K = plane_consts(A.S, of);
         Kg = grid_consts<KIND>(A.S, K);
       }

@@ -1245,7 +1245,7 @@ __global__ void k_torque_to_euler(const double* torque, const float* rotations, 
 // Response matrix: each block owns one source at a time, accumulates its
 // image row in LDS over every (facet, sample), then writes the full row
 // (render.py:271-324).  World samples come from the precomputed SoA.
-template <int SRC, int KIND, int SPLAT>
+template <int SRC, int KIND, int SPLAT, int OBST>
 __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_response(TraceArgs A) {
   extern __shared__ float smem[];
   const int P = A.S.n_pixels;
@@ -1285,7 +1285,7 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_response(TraceArgs A) 
       set_facet(smp, facet_cull(A, f, s >> 6));
       float gu, gv, v, x, y;
       const bool ok =
-          trace_ray<SRC, KIND, true, false>(A, smp, active, e, qs, val, gu, gv, v, x, y);
+          trace_ray<SRC, KIND, true, false, OBST>(A, smp, active, e, qs, val, gu, gv, v, x, y);
       if (!SPLAT) {
         const int pix = grid_pixel<KIND>(A.S, table, gu, gv, ok);
         if (A.lds_image)
@@ -1426,6 +1426,10 @@ static TraceKernel pick_trace_t(const TraceArgs& A) {
     return ob ? k_trace<SRC, KIND, SPLAT, MODE, false, 1>
               : k_trace<SRC, KIND, SPLAT, MODE, false, 0>;
   }
+  // (shadow code in a scene without obstructions costs scalar registers, which
+  // the stages' loops then spill)
+  if (MODE == IACT_MODE_IMAGE && !has_obstructions(A.ob))
+    return k_trace<SRC, KIND, SPLAT, MODE, true, 0>;
   return k_trace<SRC, KIND, SPLAT, MODE, true, 2>;
 }
 
@@ -1440,16 +1444,21 @@ static TraceKernel pick_sm_t(const TraceArgs& A) {
   return ob ? k_trace_sm<SRC, KIND, SPLAT, 1, 1> : k_trace_sm<SRC, KIND, SPLAT, 0, 1>;
 }
 
+template <int SRC, int KIND, int SPLAT>
+static TraceKernel pick_rows(const TraceArgs& A) {
+  return has_obstructions(A.ob) ? k_trace_response<SRC, KIND, SPLAT, 1>
+                                : k_trace_response<SRC, KIND, SPLAT, 0>;
+}
+
 template <int SRC>
 static TraceKernel pick_src(const TraceArgs& A, int which) {
   const bool sq = A.S.kind == IACT_SENSOR_SQUARE;
   const bool sp = A.S.splat != 0;
   switch (which) {
     case TRACE_RESPONSE:
-      if (sq) return sp ? k_trace_response<SRC, IACT_SENSOR_SQUARE, 1>
-                        : k_trace_response<SRC, IACT_SENSOR_SQUARE, 0>;
-      return sp ? k_trace_response<SRC, IACT_SENSOR_HEX, 1>
-                : k_trace_response<SRC, IACT_SENSOR_HEX, 0>;
+      if (sq) return sp ? pick_rows<SRC, IACT_SENSOR_SQUARE, 1>(A)
+                        : pick_rows<SRC, IACT_SENSOR_SQUARE, 0>(A);
+      return sp ? pick_rows<SRC, IACT_SENSOR_HEX, 1>(A) : pick_rows<SRC, IACT_SENSOR_HEX, 0>(A);
     case TRACE_DEBUG:
       return sq ? pick_trace_t<SRC, IACT_SENSOR_SQUARE, 0, IACT_MODE_DEBUG>(A)
                 : pick_trace_t<SRC, IACT_SENSOR_HEX, 0, IACT_MODE_DEBUG>(A);

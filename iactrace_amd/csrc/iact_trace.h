@@ -494,11 +494,13 @@ IACT_DEV MirrorHit mirror_hit(const TraceArgs& A, cptr<float> M, f3 ol, f3 dl) {
     z0 = sag_raw<double>(s64, x0, y0);
     z0f = sag_raw<float>(s32, M[15], M[16]);
   }
+  const bool own_sheet = conic && s64.K <= 0.0;
   const double t0 = intersect_conic((double)ol.x + x0, (double)ol.y + y0, (double)ol.z + z0,
                                     (double)dl.x, (double)dl.y, (double)dl.z, s64.c, s64.k,
-                                    conic && s64.K <= 0.0);
+                                    own_sheet);
   bool ok;
-  const double t = newton_t(s64, ol.x, ol.y, ol.z, dl.x, dl.y, dl.z, x0, y0, z0, t0, ok);
+  const double t =
+      newton_t(s64, ol.x, ol.y, ol.z, dl.x, dl.y, dl.z, x0, y0, z0, t0, own_sheet, ok);
   MirrorHit h;
   const float xh = (float)((double)ol.x + t * (double)dl.x);
   const float yh = (float)((double)ol.y + t * (double)dl.y);
@@ -530,7 +532,7 @@ struct StageRec {
 // (first minimum wins, table is ordered by group then index), reflect, and
 // value *= hit * shadow * |cos|.  A miss keeps point 0 / normal 0.  Fills rec
 // when REC.
-template <bool REC>
+template <bool REC, int OBST>
 IACT_DEV void stage_forward(const TraceArgs& A, int stage, f3& o, f3& d, float& v, bool active,
                             StageRec& rec) {
   float best = __builtin_inff();
@@ -557,7 +559,8 @@ IACT_DEV void stage_forward(const TraceArgs& A, int stage, f3& o, f3& d, float& 
   const float c = dot(d, bn);
   const f3 r = fma3(-2.f * c, bn, d);
   const float hit = best < 1e10f ? 1.f : 0.f;
-  const float shadow = has_obstructions(A.ob) ? shadow_factor(A.ob, o, d, active) : 1.f;
+  const float shadow =
+      OBST && has_obstructions(A.ob) ? shadow_factor(A.ob, o, d, active) : 1.f;
   if (REC) {
     rec.o = o;
     rec.r = d;
@@ -574,10 +577,11 @@ IACT_DEV void stage_forward(const TraceArgs& A, int stage, f3& o, f3& d, float& 
   d = r;
 }
 
+template <int OBST>
 IACT_DEV void reflect_at_stage(const TraceArgs& A, int stage, f3& o, f3& d, float& v,
                                bool active) {
   StageRec unused;
-  stage_forward<false>(A, stage, o, d, v, active, unused);
+  stage_forward<false, OBST>(A, stage, o, d, v, active, unused);
 }
 
 // Shadow factor of the primary leg: obstructions between the sample and
@@ -888,7 +892,7 @@ IACT_DEV bool trace_ray(const TraceArgs& A, const Sample& s, bool active, f3 e, 
   } else {
     f3 r = fma3(cu, s.n, u);
     f3 o = s.p;
-    for (int k = 0; k < A.n_stages; ++k) reflect_at_stage(A, A.stages[k], o, r, v, active);
+    for (int k = 0; k < A.n_stages; ++k) reflect_at_stage<OBST>(A, A.stages[k], o, r, v, active);
     const PlaneK K = plane_consts(A.S, o);
     const GridK G = grid_consts<KIND>(A.S, K);
     ok = plane_grid<KIND, AXIS, true>(A.S, G, r, gu, gv, 1.f);

@@ -289,7 +289,9 @@ IACT_DEV void stage_adjoint(const AdjArgs& B, const StageRec& rec, f3& go, f3& g
 // instance, are produced.
 // AXIS: the sensor frame is the world frame (the binning then reads the
 // direction's components instead of three dot products), as in the forward.
-template <int SRC, int KIND, int SPLAT, bool BATCH, bool STAGES, bool AXIS>
+// OBST: as in primary_shadow; without obstructions the shadow code's scalar
+// registers are free for the source loop, which otherwise spills.
+template <int SRC, int KIND, int SPLAT, bool BATCH, bool STAGES, bool AXIS, int OBST>
 __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_adj(AdjArgs B) {
   const TraceArgs& A = B.T;
   extern __shared__ float smem[];
@@ -404,7 +406,7 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_adj(AdjArgs B) {
       const f3 d = primary_direction<SRC>(smp, e, qs, inv);
       const float c = dot(d, smp.n);
       const f3 r = fma3(-2.f * c, smp.n, d);
-      const float shadow = primary_shadow<2>(A, smp, d, active);
+      const float shadow = primary_shadow<OBST>(A, smp, d, active);
       const float vunit = active ? c * smp.nrw * shadow : 0.f;  // ray value / source value
       // stages >= 1 (render.py:44-79), recorded for their adjoint
       f3 of = smp.p, rf = r;
@@ -415,7 +417,7 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_adj(AdjArgs B) {
       if (STAGES) {
 #pragma unroll
         for (int k = 0; k < IACT_ADJ_MAX_STAGES; ++k)
-          if (k < A.n_stages) stage_forward<true, 2>(A, A.stages[k], of, rf, vf, active, rec[k]);
+          if (k < A.n_stages) stage_forward<true, OBST>(A, A.stages[k], of, rf, vf, active, rec[k]);
         K = plane_consts(A.S, of);
         Kg = grid_consts<KIND>(A.S, K);
       }
@@ -631,18 +633,20 @@ __global__ __launch_bounds__(IACT_MAX_BLOCK) void k_trace_adj(AdjArgs B) {
 
 using AdjKernel = void (*)(AdjArgs);
 
-template <int SRC, int KIND, int SPLAT, bool AXIS>
-static AdjKernel pick_adj_ax(const AdjArgs& B) {
-  if (B.T.item_prefix) return k_trace_adj<SRC, KIND, SPLAT, true, false, AXIS>;
-  return B.T.n_stages > 0 ? k_trace_adj<SRC, KIND, SPLAT, false, true, AXIS>
-                          : k_trace_adj<SRC, KIND, SPLAT, false, false, AXIS>;
+template <int SRC, int KIND, int SPLAT, int OBST>
+static AdjKernel pick_adj_ob(const AdjArgs& B) {
+  // (primary hits are binned by grid_hit, splat sensors bin through plane_xy:
+  // neither has an axis variant)
+  if (B.T.n_stages == 0) return k_trace_adj<SRC, KIND, SPLAT, false, false, false, OBST>;
+  return B.T.S.axis && !SPLAT ? k_trace_adj<SRC, KIND, SPLAT, false, true, !SPLAT, OBST>
+                              : k_trace_adj<SRC, KIND, SPLAT, false, true, false, OBST>;
 }
 
 template <int SRC, int KIND, int SPLAT>
 static AdjKernel pick_adj_t(const AdjArgs& B) {
-  // splat sensors bin through plane_xy, which has no axis variant
-  return (B.T.S.axis && !SPLAT) ? pick_adj_ax<SRC, KIND, SPLAT, true>(B)
-                                : pick_adj_ax<SRC, KIND, SPLAT, false>(B);
+  if (B.T.item_prefix) return k_trace_adj<SRC, KIND, SPLAT, true, false, false, 2>;
+  return has_obstructions(B.T.ob) ? pick_adj_ob<SRC, KIND, SPLAT, 1>(B)
+                                  : pick_adj_ob<SRC, KIND, SPLAT, 0>(B);
 }
 
 template <int SRC>

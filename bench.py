@@ -11,7 +11,7 @@ the whole iteration (a ray = one (source, facet, sample) triple, traced
 forward and backward).  Inputs are resident in HBM before timing starts.
 
 Also reported:
-  * roofline of the dominant kernel, the source-major adjoint k_adj_sm
+  * roofline of the dominant kernel, the spot tree's walk k_tree
     (per instance): its algorithmic FP32 flops per batched backward (rays x
     2 x the forward's FP32 flops per ray, the backward's share under the
     fwd+bwd = 3 x fwd convention, no credit for obstruction tests) over its
@@ -176,7 +176,7 @@ def c5(ia, configs, n_instances, steps, warmup, want_parity, want_plain):
                            "the 12 FP64 flops of a point source's direction not counted"}
     peak_note = ("157.3 TFLOP/s assumes packed FP32 (two FMAs per lane per instruction); these "
                  "kernels are built without packed FP32.  frac counts algorithmic flops, which "
-                 "include work the kernels do once per facet and source instead of per ray, "
+                 "include work the kernels do once per run of samples and source instead of per ray, "
                  "and the adjoint at twice the forward's flops (so its frac can exceed 1); "
                  "valu_issue (rocprofv3 counters: VALU instructions x 4 cycles / (SIMDs x "
                  "cycles)) is the hardware's measured utilisation")
@@ -191,10 +191,10 @@ def c5(ia, configs, n_instances, steps, warmup, want_parity, want_plain):
                 "fp32_flops_per_ray": flops, "peak_note": peak_note,
                 "valu_issue": profile_value(counters, "valu_issue_frac")}
 
-    fwd_roof = roof(fwd_tf, f_ms, "k_trace_sm", "source-major forward",
-                    "k_trace_sm_C5_counters.txt", "kernel_ms_per_forward")
-    adj_roof = roof(bwd_tf, b_ms, "k_adj_sm", "source-major adjoint",
-                    "k_adj_sm_C5_counters.txt", "kernel_ms_per_backward")
+    fwd_roof = roof(fwd_tf, f_ms, "k_tree", "image walk of the spot tree",
+                    "k_tree_C5_forward_counters.txt", "kernel_ms_per_forward")
+    adj_roof = roof(bwd_tf, b_ms, "k_tree", "gradient walk of the spot tree",
+                    "k_tree_C5_adjoint_counters.txt", "kernel_ms_per_backward")
     out = {
         "value": n / it_s, "ms_per_step": 1e3 * it_s, "rays_per_step": n,
         "event_ms_per_step": float(np.mean(ev)),
@@ -337,11 +337,11 @@ def c2_forward(ia, configs, steps, warmup, want_parity):
                        "32x30 camera",
            "rays_per_step": wl.n_rays, "steps": steps, "fwd_rays_per_s": wl.n_rays * steps / wall,
            "fwd_ms": 1e3 * wall / steps,
-           "roofline": {"kernel": "k_sample_records + k_trace_sm (HIP events around the render)",
+           "roofline": {"kernel": "k_sample_records + k_tree_nodes + k_tree (HIP events around the render)",
                         "kernel_ms": k_ms, "fp32_flops_per_ray": f32,
                         "achieved_tflops": wl.n_rays * f32 / (k_ms * 1e-3) / 1e12,
                         "frac": wl.n_rays * f32 / (k_ms * 1e-3) / PEAK_FP32,
-                        "traffic": profile_value("k_trace_sm_C2_traffic.txt",
+                        "traffic": profile_value("k_tree_C2_traffic.txt",
                                                  "hbm_bytes_per_launch")}}
     if want_parity:
         from tests.helpers import oracle_scene

@@ -113,3 +113,23 @@ def test_splat_gradients_per_source(ns):
     assert float((g.double() - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
     one = torch.autograd.grad(ia.render(tel, x[-1:], v[-1:], light), x, cot)[0][-1]
     assert float((gx[-1] - one).abs().max()) <= 1e-4 * float(one.abs().max())
+
+
+@pytest.mark.parametrize("ns", [128, 1024, 1025, 4096, 4097])
+def test_sorted_sources_are_a_permutation(ns):
+    """Obstructed images sort their sources, up to 4096 in one block: the image is
+    the sum of the rays (2e-5: see test_gpu_tree), the gradients of the values come
+    back in the caller's order."""
+    tel = _telescope(16, _sensor("hex"), "all", n=3)
+    src, val, light = _sources(ns, "far", ns)
+    src, val = torch.as_tensor(src, device=DEV), torch.as_tensor(val, device=DEV)
+    P = tel.sensors[0].n_pixels
+    v = val.clone().requires_grad_(True)
+    img = ia.render(tel, src, v, light)
+    rows = _debug_rows(tel, src, torch.ones_like(val), light, ns, P)
+    ref = val.double() @ rows
+    assert float((img.detach().double() - ref).abs().max()) <= 2e-5 * float(ref.max())
+    cot = torch.rand(P, generator=torch.Generator().manual_seed(2)).to(DEV)
+    g = torch.autograd.grad(img, v, cot)[0].double()
+    want = rows @ cot.double()
+    assert float((g - want).abs().max()) <= 1e-5 * float(want.abs().max())

@@ -133,3 +133,25 @@ def test_sorted_sources_are_a_permutation(ns):
     g = torch.autograd.grad(img, v, cot)[0].double()
     want = rows @ cot.double()
     assert float((g - want).abs().max()) <= 1e-5 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("sensor", ["square", "oblong-edge-tilted", "hex", "hex-edge"])
+@pytest.mark.parametrize("samples,ns,light", [(1, 64, "far"), (65, 130, "parallel"),
+                                              (1030, 513, "far"), (100, 70, "near")])
+def test_tree_without_obstructions_by_choice(sensor, samples, ns, light):
+    """Small clear scenes take the tree where the caller asks for the source-major
+    layout (tolerances: test_gpu_tree)."""
+    s = _sensor(sensor)
+    L = ia.LaunchConfig(layout=2)
+    tel = _telescope(samples, s, "none", n=5)
+    src, val, light = _sources(ns, light, samples)
+    src, val = torch.as_tensor(src, device=DEV), torch.as_tensor(val, device=DEV)
+    v = val.clone().requires_grad_(True)
+    img = ia.render(tel, src, v, light, launch=L).reshape(-1)
+    rows = _debug_rows(tel, src, torch.ones_like(val), light, ns, s.n_pixels)
+    ref = val.double() @ rows
+    assert float((img.detach().double() - ref).abs().max()) <= 2e-5 * float(ref.max())
+    cot = torch.rand(s.n_pixels, generator=torch.Generator().manual_seed(2)).to(DEV)
+    g = torch.autograd.grad(img, v, cot)[0].double()
+    want = rows @ cot.double()
+    assert float((g - want).abs().max()) <= 1e-5 * float(want.abs().max())

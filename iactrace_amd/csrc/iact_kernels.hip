@@ -1322,8 +1322,8 @@ template <int SRC, int KIND, int OBST>
 __global__ __launch_bounds__(IACT_RESPONSE_BLOCK) void k_response(TraceArgs A) {
   extern __shared__ double rows[];
   const int P = A.S.n_pixels, T = A.resp_tile;
-  const int tile = (int)fdiv(blockIdx.x, A.d_parts), part = blockIdx.x - tile * A.resp_parts;
-  const int s0 = tile * T, n_src = min(T, A.ns - s0);
+  const int bt = (int)fdiv(blockIdx.x, A.d_parts), part = blockIdx.x - bt * A.resp_parts;
+  const int s0 = (A.resp_first + bt) * T, n_src = min(T, A.ns - s0);
   for (int i = threadIdx.x; i < n_src * P; i += IACT_RESPONSE_BLOCK) rows[i] = 0.0;
   int32_t* tab_lds = (int32_t*)(rows + T * P);
   const int32_t* table = KIND == IACT_SENSOR_HEX ? stage_hex_table(A.S, tab_lds) : tab_lds;
@@ -1512,12 +1512,22 @@ hipError_t launch_response(const TraceArgs& A, int source_type, hipStream_t st) 
   const size_t tab = A.S.kind == IACT_SENSOR_HEX
                          ? (size_t)(A.S.tq + 2) * (A.S.tr + 2) * sizeof(int32_t)
                          : 0;
-  const LaunchShape L{((A.ns + A.resp_tile - 1) / A.resp_tile) * A.resp_parts, 0,
-                      IACT_RESPONSE_BLOCK,
-                      (size_t)A.resp_tile * A.S.n_pixels * sizeof(double) + tab};
-  return launch_trace_kernel(source_type == IACT_SOURCE_POINT ? pick_response<IACT_SOURCE_POINT>(A)
-                                                              : pick_response<IACT_SOURCE_PARALLEL>(A),
-                             A, L, st);
+  const TraceKernel k = source_type == IACT_SOURCE_POINT ? pick_response<IACT_SOURCE_POINT>(A)
+                                                         : pick_response<IACT_SOURCE_PARALLEL>(A);
+  // a grid holds fewer than 2^32 threads (beyond, it would wrap): the tiles go
+  // out in launches of so many
+  const long long tiles = ((long long)A.ns + A.resp_tile - 1) / A.resp_tile;
+  const long long most = ((1ll << 32) - 1) / IACT_RESPONSE_BLOCK / A.resp_parts;
+  TraceArgs a = A;
+  for (long long t = 0; t < tiles; t += most) {
+    const long long n = tiles - t < most ? tiles - t : most;
+    a.resp_first = (int)t;
+    const LaunchShape L{(int)(n * A.resp_parts), 0, IACT_RESPONSE_BLOCK,
+                        (size_t)A.resp_tile * A.S.n_pixels * sizeof(double) + tab};
+    const hipError_t e = launch_trace_kernel(k, a, L, st);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 template <int SRC, int KIND, int SPL>

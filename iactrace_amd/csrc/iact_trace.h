@@ -109,8 +109,8 @@ struct TraceArgs {
   float* partials;
   const float* world;  // SoA (7, nf*M) when precomputed
   // response matrix from sample records (k_response): sources per block (0: not
-  // taken), parts of the sample chunks
-  int resp_tile, resp_parts;
+  // taken), parts of the sample chunks, the launch's first tile
+  int resp_tile, resp_parts, resp_first;
   FastDiv d_parts;
   int lds_image;       // image accumulated in LDS: 1 fp32, 2 fp64
   int lds_table;       // hex table staged in LDS

@@ -155,3 +155,24 @@ def test_tree_without_obstructions_by_choice(sensor, samples, ns, light):
     g = torch.autograd.grad(img, v, cot)[0].double()
     want = rows @ cot.double()
     assert float((g - want).abs().max()) <= 1e-5 * float(want.abs().max())
+
+
+def test_response_of_more_sources_than_one_grid_holds():
+    """2^24 sources and some more: blocks of 512 threads for two sources each would
+    be a grid of over 2^32 threads.  Every source has the same direction, so each
+    row is the first source's scaled by the value (three roundings: 4e-7)."""
+    groups = [g.to(DEV) for g in ia.group_mirrors(configs.parabolic_dish()[:1])]
+    groups[0] = ia.MCIntegrator(1).sample_group(groups[0], 3)
+    tel = ia.Telescope(groups, [], [ia.SquareSensor([0, 0, 36.0], [0, 0, 0], 2, 2,
+                                                    (-0.5, 0.5, -0.5, 0.5))])
+    ns = (1 << 24) + 1029
+    src = torch.tensor([[0.001, 0.002, -1.0]], dtype=torch.float64, device=DEV).repeat(ns, 1)
+    val = torch.linspace(0.5, 1.5, ns, dtype=torch.float32, device=DEV)
+    row = ia.render_response_matrix(tel, src[:1], torch.ones(1, device=DEV), "parallel")
+    assert float(row.max()) > 0
+    got = ia.render_response_matrix(tel, src, val, "parallel")
+    err = 0.0
+    for a in range(0, ns, 1 << 22):
+        want = val[a:a + (1 << 22), None] * row
+        err = max(err, float((got[a:a + (1 << 22)] - want).abs().max()))
+    assert err <= 4e-7 * 1.5 * float(row.max())

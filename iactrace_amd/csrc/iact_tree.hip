@@ -848,7 +848,9 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
       if (OBST && valid) dsum = dsum - ie * e;
     }
     // ---- obstruction candidates of the item: those the cone of its sources'
-    // directions (with the parallax of near ones) can reach from the top's ball
+    // directions (with the parallax of near ones: a ray's direction is e + q,
+    // |q| at most the distance of the top's farthest sample from the facet
+    // position) can reach from the top's ball
     const f3 tc = mk3(tball[0], tball[1], tball[2]);
     const float trho = tball[3];
     f3 ax = mk3(0.f, 0.f, 1.f);
@@ -870,6 +872,8 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
       // the largest tan(angle + parallax), from the chord (acos of a cosine
       // next to 1 would be off by 3e-4 rad); beyond 80 degrees: no culling
       float tg = 0.f;
+      const f3 tq = tc - pos;
+      const float qmax = trho + 1.0001f * fsqrt(dot(tq, tq));
 #pragma unroll
       for (int r = 0; r < NS; r += NT) {
         const int si = r + tid;
@@ -879,7 +883,7 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
         const float c2 = dot(ch, ch), cs = fmaf(-0.5f, c2, 1.f);
         float g = cs > 0.17f ? fsqrt(c2 * fmaf(-0.25f, c2, 1.f)) * frcp(cs) : 1e30f;
         if (SRC == IACT_SOURCE_POINT) {
-          const float sp = trho * ie, cp2 = fmaf(-sp, sp, 1.f);
+          const float sp = qmax * ie, cp2 = fmaf(-sp, sp, 1.f);
           const float tp = cp2 > 0.03f ? sp * frsq(cp2) : 1e30f;
           g = g * tp < 0.9f ? (g + tp) * frcp(fmaf(-g, tp, 1.f)) : 1e30f;
         }

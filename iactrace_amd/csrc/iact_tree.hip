@@ -570,7 +570,7 @@ __global__ __launch_bounds__(256) void k_tree_nodes(TraceArgs A, TreeParams K, f
 template <int MODE>
 struct TreeLds {
   using Img = std::conditional_t<MODE == 0, double, float>;
-  static constexpr uint32_t src = 0;  // e, value / |u|, da, db (, 1 / |u|)
+  static constexpr uint32_t src = 0;  // u, value / |u|, da, db (, 1 / |e|): see scaled_inv
   static constexpr uint32_t l0 = src + (MODE == 2 ? 7u : 6u) * kTreeSources * 4u;
   static constexpr uint32_t wl = l0 + kTreeSources * 2u;
   static constexpr uint32_t pc = wl + kWaves * 2u * kTreeSources * 2u;
@@ -740,6 +740,17 @@ IACT_DEV uint32_t shade_bits(const iact_obstructions& ob, int j, f3 myp, int nq,
   return bits;
 }
 
+// A far point source's u is kept as e times the power of two 2^x that brings |u|
+// to (1, 2], with 1 / |e| = 2^x / |u|.  No decision and no term of a ray changes but
+// by that power, and value / |u| keeps fp32's range: at |e| = 1e10 m, value / |e| of
+// a flux of 1e-29 is subnormal, and so is its product with a small image gradient
+// (rotation gradients of fluxes and image gradients of 2^-55 were off by 0.6 of the
+// largest, ray by ray 2e-6).
+IACT_DEV float scaled_inv(float ie) { return __builtin_amdgcn_frexp_mantf(ie); }  // 1 / |u|
+IACT_DEV float per_metre(float v, float ie) {                                     // v 2^x
+  return __builtin_ldexpf(v, __builtin_amdgcn_frexp_expf(ie));
+}
+
 // A work item is a block of kTreeSources sources against one top of a facet.
 // The block's threads test the top for one source each and list the sources it
 // does not resolve; each wave then takes patches of the top, tests the listed
@@ -830,21 +841,27 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
       const double* sp = A.sources + 3 * (size_t)sl;
       const f3 e = source_offset<SRC>(sp[0], sp[1], sp[2], pos);
       const float value = valid ? A.values[sl] : 0.f;
-      const float ie = frsq(dot(e, e)), inv = SRC == IACT_SOURCE_POINT ? ie : 1.f;
+      const float ie = frsq(dot(e, e));
       const bool far = valid && (SRC != IACT_SOURCE_POINT || source_qs(A, e) == 0.f);
+      const bool scaled = SRC == IACT_SOURCE_POINT && far;
+      const float pw = scaled ? per_metre(1.f, ie) : 1.f;
+      const float vi =
+          value * (SRC == IACT_SOURCE_POINT ? (scaled ? scaled_inv(ie) : ie) : 1.f);
       const f3 U = sensor_dirs(A.S, e);
       const float iu = frcp(U.x);
       float da = fmaf(U.y, iu, -a0);
-      const float db = fmaf(U.z, iu, -b0);
-      if (!(far && U.x * ie * sign > 1e-3f && fabsf(da) + fabsf(db) <= tau))
-        da = __builtin_nanf("");
-      sx[si] = e.x;
-      sy[si] = e.y;
-      sz[si] = e.z;
-      svi[si] = value * inv;
+      float db = fmaf(U.z, iu, -b0);
+      if (!(far && U.x * ie * sign > 1e-3f && fabsf(da) + fabsf(db) <= tau)) {
+        da = __builtin_nanf("");     // no node's test resolves it
+        db = far ? 0.f : da;         // (NaN: not far)
+      }
+      sx[si] = pw * e.x;
+      sy[si] = pw * e.y;
+      sz[si] = pw * e.z;
+      svi[si] = vi;
       sda[si] = da;
       sdb[si] = db;
-      if (MODE == 2) sinv[si] = inv;
+      if (MODE == 2) sinv[si] = SRC == IACT_SOURCE_POINT ? ie : 1.f;
       if (OBST && valid) dsum = dsum - ie * e;
     }
     // ---- obstruction candidates of the item: those the cone of its sources'
@@ -882,7 +899,7 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
         const f3 ch = -ie * e - ax;
         const float c2 = dot(ch, ch), cs = fmaf(-0.5f, c2, 1.f);
         float g = cs > 0.17f ? fsqrt(c2 * fmaf(-0.25f, c2, 1.f)) * frcp(cs) : 1e30f;
-        if (SRC == IACT_SOURCE_POINT) {
+        if (SRC == IACT_SOURCE_POINT && !(sdb[si] == sdb[si])) {  // (far: below 2^-30)
           const float sp = qmax * ie, cp2 = fmaf(-sp, sp, 1.f);
           const float tp = cp2 > 0.03f ? sp * frsq(cp2) : 1e30f;
           g = g * tp < 0.9f ? (g + tp) * frcp(fmaf(-g, tp, 1.f)) : 1e30f;
@@ -939,10 +956,11 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
         const float g = img[pix], w = g * vi;
         Aw = fma3(w, u, Aw);
         if (MODE == 2) {
-          const float i1 = sinv[si];
+          const float ie = sinv[si], i1 = SRC == IACT_SOURCE_POINT ? scaled_inv(ie) : 1.f;
           if (want_pos && SRC == IACT_SOURCE_POINT) {
-            w1 += w;
-            Dw = fma3(w * us * (i1 * i1), u, Dw);
+            const float wm = per_metre(w, ie);
+            w1 += wm;
+            Dw = fma3(wm * us * (i1 * i1), u, Dw);
           }
           if (want_val) lds_add(acc + si, g * (us * i1));
           if (want_src) {
@@ -999,7 +1017,7 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
       const int si = r + tid;
       const bool valid = sb * NS + si < A.ns;
       const f3 e = mk3(sx[si], sy[si], sz[si]);
-      const bool far = valid && (SRC != IACT_SOURCE_POINT || source_qs(A, e) == 0.f);
+      const bool far = valid && (SRC != IACT_SOURCE_POINT || sdb[si] == sdb[si]);
       bool sus = false;
       if (OBST && nlc > 0) {
         if (nlc <= 64 && !A.cull_all) {
@@ -1078,8 +1096,10 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
       auto add_rays = [&](f3 N, f3 u, float vi, int si) {
         T = T + vi * cross(N, u);
         if (MODE == 2) {
-          const float i1 = sinv[si], un = dot(u, N) * i1;
-          if (want_pos && SRC == IACT_SOURCE_POINT) Gp = Gp + vi * fma3(-un * i1, u, N);
+          const float ie = sinv[si], i1 = SRC == IACT_SOURCE_POINT ? scaled_inv(ie) : 1.f;
+          const float un = dot(u, N) * i1;
+          if (want_pos && SRC == IACT_SOURCE_POINT)
+            Gp = Gp + per_metre(vi, ie) * fma3(-un * i1, u, N);
           if (want_val) lds_add(acc + si, un);
           if (want_src) {
             lds_add(acc + NS + si, N.x);
@@ -1430,11 +1450,13 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
       if (want_val && acc[si] != 0.0) unsafeAtomicAdd(B.g_val + so, acc[si]);
       if (want_src) {
         const f3 N = mk3((float)acc[NS + si], (float)acc[2 * NS + si], (float)acc[3 * NS + si]);
-        const f3 e = mk3(sx[si], sy[si], sz[si]), d = sinv[si] * e;
+        const f3 d = scaled_inv(sinv[si]) * mk3(sx[si], sy[si], sz[si]);
         // far: dL/dsrc = -value / |u| (N - (d.N) d); near sources have theirs
         // summed already; parallel: value N (1 / |u| is 1)
         const f3 g = SRC == IACT_SOURCE_POINT
-                         ? (source_qs(A, e) == 0.f ? (-svi[si]) * fma3(-dot(d, N), d, N) : N)
+                         ? (sdb[si] == sdb[si]
+                                ? per_metre(-svi[si], sinv[si]) * fma3(-dot(d, N), d, N)
+                                : N)
                          : svi[si] * N;
         unsafeAtomicAdd(B.g_src + 3 * so, (double)g.x);
         unsafeAtomicAdd(B.g_src + 3 * so + 1, (double)g.y);

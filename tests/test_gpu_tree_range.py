@@ -1,0 +1,56 @@
+"""The spot tree's numbers at the ends of fp32, on the GPU.
+
+Renders are linear in the sources' values and their gradients in values and
+image gradients, so powers of two come back exactly wherever no intermediate
+leaves fp32's range; what is left is the order of the sums (1e-6 of the largest,
+of some 10^2 fp32 additions each 2^-24).
+"""
+import pytest
+import torch
+
+import iactrace_amd as ia
+from tests.test_gpu_tree import _sensor, _sources, _telescope
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _all(tel, src, val, st, cot, layout=0):
+    g = tel.mirror_groups[0]
+    leaves = [t.detach().clone().requires_grad_(True)
+              for t in (g.rotations, g.positions, src, val)]
+    rot, pos, s, v = leaves
+    t = ia.Telescope([g.replace(rotations=rot, positions=pos)], tel.obstruction_groups,
+                     tel.sensors)
+    img = ia.render(t, s, v, st, launch=ia.LaunchConfig(layout=layout)).reshape(-1)
+    grads = torch.autograd.grad(img, leaves, cot)
+    return dict(zip(("image", "rotations", "positions", "sources", "values"),
+                    [x.detach().double() for x in (img, *grads)]))
+
+
+def _scene(light):
+    tel = _telescope(100, _sensor("hex"), "all", 0.0, 5, n_facets=7)
+    src, val, st = _sources(300, light, 3)
+    cot = torch.linspace(0.5, 1.5, tel.sensors[0].n_pixels, device=DEV)
+    return tel, torch.as_tensor(src, device=DEV), torch.as_tensor(val, device=DEV), st, cot
+
+
+@pytest.mark.parametrize("light", ["far", "near", "parallel"])
+@pytest.mark.parametrize("a,b,per_metre", [(2.0 ** -60, 1.0, True), (2.0 ** -100, 1.0, False),
+                                           (2.0 ** -55, 2.0 ** -55, False),
+                                           (2.0 ** 60, 2.0 ** 60, True)])
+def test_powers_of_two_come_back(light, a, b, per_metre):
+    """a: of the values, b: of the image gradient.  per_metre: with the gradients
+    per metre, which are smaller by the distance (2^33 at 1e10 m, 2^13 near by):
+    ones that leave fp32's range themselves are not compared."""
+    tel, src, val, st, cot = _scene(light)
+    base = _all(tel, src, val, st, cot)
+    got = _all(tel, src, val * a, st, cot * b)
+    factor = {"image": a, "rotations": a * b, "positions": a * b, "sources": a * b, "values": b}
+    for k, f in factor.items():
+        if k in ("positions", "sources") and not per_metre:
+            continue
+        scale = float(base[k].abs().max())
+        err = float((got[k] / f - base[k]).abs().max())
+        print(f"[range {light} {a:.1e} {b:.1e}] {k}: {err / max(scale, 1e-300):.1e}", flush=True)
+        assert err <= 1e-6 * scale, k

@@ -829,6 +829,8 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
     if (MODE == 2) {
       for (int i = tid; i < K.n_acc * NS; i += NT) acc[i] = 0.0;
     }
+    f3 T = mk3(0.f, 0.f, 0.f), Gp = mk3(0.f, 0.f, 0.f);  // lane's torque and dL/dpos
+    constexpr float inf = __builtin_inff();
     // ---- the item's sources
     const cptr<float> fp = as_const(A.positions) + 3 * f;
     const f3 pos = mk3(fp[0], fp[1], fp[2]);
@@ -851,9 +853,14 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
       const float iu = frcp(U.x);
       float da = fmaf(U.y, iu, -a0);
       float db = fmaf(U.z, iu, -b0);
-      if (!(far && U.x * ie * sign > 1e-3f && fabsf(da) + fabsf(db) <= tau)) {
-        da = __builtin_nanf("");     // no node's test resolves it
-        db = far ? 0.f : da;         // (NaN: not far)
+      // a value that is not finite spreads as it does ray by ray: to every pixel
+      // that one of its rays meets, shaded or not, and to every facet's gradients
+      const bool finite = MODE || fabsf(vi) < inf;
+      if (MODE && far) T = T + mk3(0.f * vi, 0.f * vi, 0.f * vi);
+      if (MODE == 2 && scaled) Gp = Gp + mk3(0.f * vi, 0.f * vi, 0.f * vi);
+      if (!(far && finite && U.x * ie * sign > 1e-3f && fabsf(da) + fabsf(db) <= tau)) {
+        da = __builtin_nanf("");                // no node's test resolves it
+        db = !far ? da : (finite ? 0.f : inf);  // (NaN: not far, inf: not shaded)
       }
       sx[si] = pw * e.x;
       sy[si] = pw * e.y;
@@ -942,7 +949,6 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
       }
       return sus;
     };
-    f3 T = mk3(0.f, 0.f, 0.f), Gp = mk3(0.f, 0.f, 0.f);  // lane's torque and dL/dpos
     f3 Aw = mk3(0.f, 0.f, 0.f), Dw = mk3(0.f, 0.f, 0.f);
     float w1 = 0.f;
     // a pair resolved to pixel pix adds its node's rays at once
@@ -1236,6 +1242,7 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
                 load_group(g);
                 sus |= pmask != 0ull && (A.cull_all || reached(pmask, pid, bc, brho, dn, act));
               }
+              if (MODE == 0) sus = sus && sdb[si] != inf;
             }
             int code = kUnresolved;
             if (ptest) code = node_test<KIND>(A.S, K, tab, pnode, sda[si], sdb[si]);

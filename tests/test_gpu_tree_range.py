@@ -54,3 +54,24 @@ def test_powers_of_two_come_back(light, a, b, per_metre):
         err = float((got[k] / f - base[k]).abs().max())
         print(f"[range {light} {a:.1e} {b:.1e}] {k}: {err / max(scale, 1e-300):.1e}", flush=True)
         assert err <= 1e-6 * scale, k
+
+
+@pytest.mark.parametrize("light", ["far", "near", "parallel"])
+@pytest.mark.parametrize("what", ["nan value", "inf value", "nan source", "inf source",
+                                  "nan image gradient"])
+def test_numbers_that_are_not_finite_spread_as_ray_by_ray(light, what):
+    """They reach the same pixels and gradients as in the sample-major kernels, and
+    no others (the rest: 1e-5 of the largest, see test_gpu_tree)."""
+    tel, src, val, st, cot = _scene(light)
+    bad = float(what.split()[0])
+    lit = int(_all(tel, src, val, st, cot)["image"].argmax())
+    {"value": val[17:18], "source": src[17], "image": cot[lit:lit + 1]}[what.split()[1]][:] = bad
+    ref = _all(tel, src, val, st, cot, layout=1)
+    got = _all(tel, src, val, st, cot)
+    for k in ref:
+        a, b = torch.isfinite(ref[k]), torch.isfinite(got[k])
+        print(f"[finite {light} {what}] {k}: {int((~a).sum())} not, {int((~b).sum())} here",
+              flush=True)
+        assert bool((a == b).all()), k
+        if bool(a.any()):
+            assert float((got[k] - ref[k])[a].abs().max()) <= 1e-5 * float(ref[k][a].abs().max())

@@ -1574,8 +1574,10 @@ bool tree_serves(const TraceArgs& A, int mode, int n_acc, const DevInfo& dev, La
                      : mode == 1 ? tree_lds_bytes<1>(A.S.n_pixels, tw, n_ob, 0)
                                  : tree_lds_bytes<2>(A.S.n_pixels, tw, n_ob, n_acc);
   if (lds > 65536) return false;
-  const long long items = (long long)A.nf * ((A.M + kTopSamples - 1) / kTopSamples) *
-                          ((A.ns + kTreeSources - 1) / kTreeSources);
+  // k_tree_nodes has 256 threads per (facet, top), and a grid of 2^32 threads wraps
+  const long long tops = (long long)A.nf * ((A.M + kTopSamples - 1) / kTopSamples);
+  if (tops >= (1ll << 24)) return false;
+  const long long items = tops * (((long long)A.ns + kTreeSources - 1) / kTreeSources);
   if (items >= (1ll << 27)) return false;
   // the rows (An, Au, Av) must be invertible (they are for a rotation)
   const f3 n = A.S.An, u = A.S.Au, v = A.S.Av;

@@ -5,10 +5,14 @@ image gradients, so powers of two come back exactly wherever no intermediate
 leaves fp32's range; what is left is the order of the sums (1e-6 of the largest,
 of some 10^2 fp32 additions each 2^-24).
 """
+import ctypes
+
 import pytest
 import torch
 
 import iactrace_amd as ia
+from iactrace_amd import _lib
+from iactrace_amd.render import LaunchConfig, RenderPlan
 from tests.test_gpu_tree import _sensor, _sources, _telescope
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +79,20 @@ def test_numbers_that_are_not_finite_spread_as_ray_by_ray(light, what):
         assert bool((a == b).all()), k
         if bool(a.any()):
             assert float((got[k] - ref[k])[a].abs().max()) <= 1e-5 * float(ref[k][a].abs().max())
+
+
+def test_tree_ends_where_its_grids_would_wrap():
+    """2^24 runs of 1024 samples: the nodes' kernel would need 2^32 threads.  The
+    workspace tells the kernels apart (nothing is launched): 144 bytes for each of a
+    facet's three nodes beside its record, or the culling tables alone."""
+    plan = RenderPlan(_telescope(1, _sensor("square"), "all", 0.0, 5, n_facets=7))
+    sc = plan.scene([])
+    L = LaunchConfig().abi()
+
+    def per_facet(n):
+        sc.facets.n_facets = n
+        return _lib.lib().iact_workspace_size(ctypes.byref(sc), 128, _lib.MODE_IMAGE,
+                                              ctypes.byref(L)) / n
+
+    assert per_facet((1 << 24) - 1) > 64 + 3 * 144
+    assert 64 < per_facet(1 << 24) < 64 + 3 * 144

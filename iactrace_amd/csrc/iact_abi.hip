@@ -554,7 +554,8 @@ CullLayout cull_layout(int nf, int words, int all, size_t base, const CullSpec& 
 // culling tables (256-B aligned): n_images * n_pixels doubles.
 size_t image64_offset(size_t end) { return align256(end); }
 
-// tree: the render takes the spot tree where that serves it
+// tree: an image takes the spot tree, a response matrix k_response, where they
+// serve it
 static size_t workspace_bytes_for(const iact_scene& sc, int ns, int mode, const LaunchShape& shp,
                                   const TraceArgs& A, const DevInfo& dev, bool tree) {
   LaunchShape ts;
@@ -954,10 +955,12 @@ int32_t iact_trace_fwd_noalloc(const iact_scene* scene, const double* sources,
   // per sample) takes the sample-major layout, which has none
   iact_launch L = launch ? *launch : iact_launch{};
   // (a size of 0 from an invalid launch: iact_trace_fwd reports the error);
-  // between the two lies the source-major trace without the spot tree's nodes
+  // between the two lies the source-major trace without the spot tree's nodes,
+  // and a response matrix from 28 B of world-space samples instead of 64-B
+  // records
   bool tree = true;
   size_t need = workspace_size(scene, n_sources, mode, &L, true);
-  if (need > (size_t)IACT_NOALLOC_SCRATCH_BYTES && mode == IACT_MODE_IMAGE) {
+  if (need > (size_t)IACT_NOALLOC_SCRATCH_BYTES && mode != IACT_MODE_DEBUG) {
     tree = false;
     need = workspace_size(scene, n_sources, mode, &L, false);
   }

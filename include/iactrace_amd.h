@@ -265,7 +265,8 @@ int32_t iact_trace_fwd(const iact_scene* scene, const double* sources, const flo
  * (held until the process ends) instead of a caller buffer.  Arguments,
  * outputs and errors as iact_trace_fwd; an image render whose default
  * layout needs more scratch than that (the source-major layout's record
- * table, 64 B per facet sample) runs the sample-major layout instead, and a
+ * table, 64 B per facet sample) runs the sample-major layout instead, a
+ * response matrix takes 28 B per sample instead of records' 64, and a
  * render that still does not fit fails with IACT_ERR_UNSUPPORTED.  Calls no
  * allocating routine.  Every call on a GPU shares that GPU's array: calls
  * that overlap on one GPU (on different streams or host threads) race and

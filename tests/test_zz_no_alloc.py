@@ -121,3 +121,30 @@ def test_noalloc_rejects_what_does_not_fit():
     assert rc == _lib.IACT_ERR_UNSUPPORTED
     assert b"scratch" in lib.iact_last_error()
     assert float(out.abs().sum()) == 0.0
+
+
+def test_noalloc_response_between_the_two_workspaces():
+    # 875 x 1024 samples: 57 MB of sample records, 25 MB of world-space samples
+    plan, src, val, st = _inputs("C3", 40, 1024)
+    keep = [src, val]
+    sc = plan.scene(keep)
+    L = LaunchConfig().abi()
+    lib = _lib.lib()
+    need = lib.iact_workspace_size(ctypes.byref(sc), 40, _lib.MODE_RESPONSE, ctypes.byref(L))
+    assert need > _lib.IACT_NOALLOC_SCRATCH_BYTES
+    P = plan.sensor.n_pixels
+    ws = torch.empty(int(need), dtype=torch.uint8, device=DEV)
+    a, b = (torch.full((40, P), -7.0, device=DEV) for _ in range(2))
+    for _ in range(2):
+        rc = lib.iact_trace_fwd_noalloc(ctypes.byref(sc), _lib.ptr(src), _lib.ptr(val), 40, st,
+                                        _lib.MODE_RESPONSE, ctypes.byref(L), _lib.ptr(a), None,
+                                        None, _lib.current_stream())
+        _lib.check(rc, "iact_trace_fwd_noalloc")
+    _lib.check(lib.iact_trace_fwd(ctypes.byref(sc), _lib.ptr(src), _lib.ptr(val), 40, st,
+                                  _lib.MODE_RESPONSE, ctypes.byref(L), _lib.ptr(ws), ws.numel(),
+                                  _lib.ptr(b), None, None, _lib.current_stream()),
+               "iact_trace_fwd")
+    scale = b.abs().amax(1, keepdim=True)
+    assert int((scale > 0).sum()) >= 3  # (the rest of the field misses the camera)
+    # (rows of fp64 sums on both sides: see test_gpu_rows)
+    assert float(((a - b).abs() / scale.clamp_min(1e-30)).max()) < 2e-6

@@ -224,6 +224,7 @@ class RenderPlan:
         ob = pack_obstruction_tables(self.tel.obstruction_groups or [])
         self.obstruction_tables = {k: torch.as_tensor(v).to(dev).contiguous() for k, v in ob.items()}
         self.sensor_abi = self.sensor.to_abi(dev)
+        self.facet_counts = [len(g) for g in self.primary]
         self.surface_index = _surface_index(self.primary, dev) if self.primary else None
         self.static_scene = self._static_scene()
 
@@ -252,6 +253,10 @@ class RenderPlan:
     def scene(self, keep, rotations=None, positions=None):
         sc = _lib.IactScene.from_buffer_copy(self.static_scene)
         if self.primary:
+            counts = [len(g) for g in self.primary]
+            if counts != self.facet_counts:  # (a group's tensors were replaced by others)
+                self.surface_index = _surface_index(self.primary, self.device)
+                self.facet_counts = counts
             sc.facets = facets_abi(self.primary, keep, rotations, positions, self.surface_index)
         for i, g in enumerate(self.surface_groups):
             sc.surfaces[i] = g.surface_abi()

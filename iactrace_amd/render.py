@@ -330,6 +330,10 @@ class RenderPlan:
         if need[4]:
             outs["aspheric"] = torch.empty((_lib.IACT_MAX_SURFACES, _lib.IACT_MAX_ASPHERIC),
                                            dtype=torch.float64, device=dev)
+        if need[4] and self.surface_index is not None:
+            # (read by the aspheric gradients alone, and made on the plan's first
+            # stream: the plan may be gone before this one is done)
+            self.surface_index.record_stream(torch.cuda.current_stream(dev))
         for k, v in outs.items():
             setattr(G, k, v.data_ptr())
         if not outs:

@@ -4,7 +4,8 @@ shapes XLA chooses).
 ``autotune(tel, sources, values, ...)`` asks the library (``iact_autotune``)
 to time candidate launch settings -- image layout (lanes = samples of one
 facet, or lanes = sources), block size, blocks per CU, source tile or sample
-group -- on the given inputs and returns the fastest as a ``LaunchConfig``;
+group; the automatic launch where it takes a kernel without such settings --
+on the given inputs and returns the fastest as a ``LaunchConfig``;
 with ``apply`` it becomes the telescope's default (``tel.launch``).  Results
 are cached in a JSON file keyed by the GPU architecture and the workload's
 shape (facets, samples, source count rounded to a power of two, sensor,
@@ -116,9 +117,10 @@ def autotune(tel, sources, values, source_type="point", sensor_idx=0, mode="imag
     sc = plan.scene(keep)
     L0 = (base or LaunchConfig()).abi()
     lib = _lib.lib()
-    # workspace for the largest candidate (the source-major layout's records)
+    # workspace for the largest candidate (the spot tree's nodes, the
+    # source-major layout's records)
     need = 0
-    for lay in (1, 2):
+    for lay in (0, 1, 2):
         Lc = (base or LaunchConfig()).abi()
         Lc.layout = lay
         need = max(need, int(lib.iact_workspace_size(ctypes.byref(sc), ns, _MODES[mode],

@@ -385,7 +385,7 @@ int shape_trace(const iact_scene& sc, int ns, int mode, const iact_launch* L, Tr
   const int lay = L ? L->layout : 0;
   if (lay < 0 || lay > 2) return set_error(IACT_ERR_INVALID, "layout %d", lay);
   A.layout = 1;
-  A.tree_any = lay == 2;
+  A.per_ray = lay == 2;
   // the source-major trace indexes samples in 31 bits
   const bool sm_fits = (long long)A.nf * A.M < (1ll << 31);
   if (mode == IACT_MODE_IMAGE && lay == 2 && (A.det || sc.n_stages > 0 || !sm_fits))
@@ -629,7 +629,7 @@ int adj_sm_layout(const iact_scene& sc, const double* sources, const float* valu
   l.layout = 2;
   int rc = shape_trace(sc, ns, IACT_MODE_IMAGE, &l, A, shp, dev, -1);
   if (rc) return rc;
-  A.tree_any = L && L->layout == 2;
+  A.per_ray = L && L->layout == 2;
   out.recs_end = base_workspace_bytes(sc, IACT_MODE_IMAGE, shp, A);
   const CullSpec c{ns, 1, nullptr, true, refine_groups(A, IACT_MODE_IMAGE)};
   const size_t end = cull_layout(A.nf, A.cull_words, A.cull_all, out.recs_end, c).end;
@@ -641,6 +641,16 @@ int adj_sm_layout(const iact_scene& sc, const double* sources, const float* valu
     if (t > out.end) out.end = t;
   }
   return IACT_OK;
+}
+
+bool fixed_launch(const iact_scene& sc, int ns, int mode, const iact_launch* L,
+                  const DevInfo& dev) {
+  TraceArgs A;
+  fill_trace_args(A, sc, nullptr, nullptr, ns);
+  LaunchShape shp, ts;
+  if (shape_trace(sc, ns, mode, L, A, shp, dev, -1)) return false;
+  return mode == IACT_MODE_RESPONSE ? A.resp_tile > 0
+                                    : mode == IACT_MODE_IMAGE && tree_serves(A, 0, 0, dev, ts);
 }
 
 bool tree_shared(const iact_scene& sc, int ns, const iact_launch* L, const DevInfo& dev) {

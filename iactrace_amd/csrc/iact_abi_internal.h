@@ -75,6 +75,10 @@ int tree_max_grid(const DevInfo& dev);
 bool tree_serves(const TraceArgs& A, int mode, int n_acc, const DevInfo& dev, LaunchShape& shp);
 int launch_tree(AdjArgs& B, const TreeLayout& T, void* workspace, const LaunchShape& shp,
                 int source_type, int mode, int n_acc, bool built, hipStream_t st);
+// Whether the launch takes a kernel that shapes itself (the spot tree,
+// k_response), whatever the launch's block size, grid, tile and sample group.
+bool fixed_launch(const iact_scene& sc, int ns, int mode, const iact_launch* L,
+                  const DevInfo& dev);
 // Whether an image launch and a rotation gradient of it both walk the tree, whose
 // preparation the second can then take over from the first; and that gradient
 // (iact_trace_bwd with tree_built).

@@ -3,7 +3,8 @@
 // reference has nothing to tune (XLA picks its own launch shapes); the
 // candidates here are the knobs that measurably matter on gfx950 -- image
 // layout (lanes = samples of a facet or lanes = sources), block size,
-// blocks per CU, and the source tile / sample group.
+// blocks per CU, and the source tile / sample group -- and, where it takes a
+// kernel of its own that has no such knobs, the automatic launch.
 #include <float.h>
 #include <string.h>
 
@@ -29,13 +30,22 @@ int32_t iact_autotune(const iact_scene* scene, const double* sources, const floa
   *best = b0;
   if (best_ms) *best_ms = -1.f;
   // candidate grid (the deterministic flag and accumulate mode are kept)
+  DevInfo dev;
+  rc = device_info(dev);
+  if (rc) return rc;
   iact_launch cand[64];
   int nc = 0;
+  iact_launch automatic = b0;
+  automatic.block_threads = automatic.source_tile = automatic.blocks_per_cu = 0;
+  automatic.layout = automatic.sample_group = 0;
+  const bool fixed = fixed_launch(*scene, n_sources, mode, &automatic, dev);
+  if (fixed) cand[nc++] = automatic;
   const int layouts[2] = {1, 2};
   const int threads[2] = {256, 128};
   const int bpcs[2] = {16, 64};
   const int tiles[2] = {64, 256};
-  for (int li = 0; li < (mode == IACT_MODE_IMAGE ? 2 : 1); ++li)
+  // (a response matrix has no other layout to choose)
+  for (int li = 0; li < (mode == IACT_MODE_IMAGE ? 2 : fixed ? 0 : 1); ++li)
     for (int ti = 0; ti < 2; ++ti)
       for (int bi = 0; bi < 2; ++bi)
         for (int si = 0; si < 2; ++si) {

@@ -131,7 +131,7 @@ struct TraceArgs {
   int xcd_order;                 // 1: XCD-major block numbering
   // source-major layout: lanes are sources, samples come from `recs`
   int layout;                    // 1 sample-major, 2 source-major
-  int tree_any;                  // source-major by the caller's choice: the tree at any size
+  int per_ray;                   // source-major by the caller's choice: ray by ray, no tree
   const float* recs;             // (nf*M, IACT_REC_WORDS) world-space sample records
   int sample_group;              // samples per work item
   int sm_spl;                    // sources per lane (1 or 2)

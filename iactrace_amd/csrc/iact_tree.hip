@@ -1555,20 +1555,20 @@ TreeLayout tree_layout(const iact_scene& sc, int ns, bool sort, int grid) {
 int tree_max_grid(const DevInfo& dev) { return dev.n_cu * (24 / kWaves); }
 
 bool tree_serves(const TraceArgs& A, int mode, int n_acc, const DevInfo& dev, LaunchShape& shp) {
-  if (A.layout != 2 || A.S.splat || A.n_stages > 0 || A.det || A.nf <= 0 || A.ns <= 0) return false;
+  if (A.layout != 2 || A.per_ray || A.S.splat || A.n_stages > 0 || A.det || A.nf <= 0 || A.ns <= 0) return false;
   if (A.S.n_pixels > 32767) return false;
   const int n_ob = n_obstructions(A.ob);
   if (n_ob > 65535) return false;
   // Fewer sources leave a block's lanes idle: gradients of 875 x 1000 samples x
   // 100 sources behind masts, 1630 us in the tree, 1180 ray by ray.
-  if (A.ns < 128 && !A.tree_any) return false;
+  if (A.ns < 128) return false;
   // Without shadows to save, the preparation and the tests (some 0.2 ns per sample
   // and top) and the tails of few items have to be repaid by runs on one pixel,
   // which rough mirrors and near sources have few of.  Images of 2e8 rays: 12 m
   // dish, 382 x 512 x 1024, mirrors of 24 arcsec, 430 us against 354; 28 m dish,
   // smooth, far, 875 x 1024 x 300: 344 against 468; gradients of 8.75e8 rays 2730
   // against 2560, rough; 6.4e9 smooth ones 1020 against 3680.
-  if (n_ob == 0 && (double)A.nf * A.M * A.ns < 1.5e9 && !A.tree_any) return false;
+  if (n_ob == 0 && (double)A.nf * A.M * A.ns < 1.5e9) return false;
   const int tw = table_words(A.S);
   const size_t lds = mode == 0   ? tree_lds_bytes<0>(A.S.n_pixels, tw, n_ob, 0)
                      : mode == 1 ? tree_lds_bytes<1>(A.S.n_pixels, tw, n_ob, 0)

@@ -161,14 +161,26 @@ typedef struct iact_launch {
                               -1 = all chunks (source tile slowest)          */
   int32_t block_order;     /* 0 = XCD-major block numbering (default),
                               1 = hardware block numbering                  */
-  int32_t layout;          /* image renders: 0 = automatic, 1 = lanes are
-                              the samples of one facet (wave-merged pixel
-                              sums; best when a wave's rays share pixels),
+  int32_t layout;          /* image renders and their adjoint:
+                              1 = lanes are the samples of one facet (wave-
+                              merged pixel sums; best when a wave's rays
+                              share pixels),
                               2 = lanes are sources, samples read from a
                               per-call world-space record table in the
-                              workspace (one LDS add per ray; best for many
-                              sources spread over the sensor)               */
-  int32_t sample_group;    /* layout 2: samples per work item (0 = 64)     */
+                              workspace, every ray traced (best for many
+                              sources spread over the sensor),
+                              0 = automatic: 1 below 64 sources and through
+                              further stages, 2 above, and from 128 sources
+                              runs of samples summed at once where they meet
+                              one pixel (hard binning; without obstructions
+                              from 1.5e9 rays).  Those runs' kernel, and the
+                              response matrix of primary-only hard-binned
+                              scenes, shape themselves: block_threads,
+                              blocks_per_cu, source_tile, sample_group,
+                              accumulate, chunk_block and block_order have
+                              no effect there                               */
+  int32_t sample_group;    /* layout 2: samples per work item (0 = 64; fewer
+                              for splat sensors where items are few)       */
   int32_t culling;         /* obstruction culling: a prepass bounds, per
                               facet, the bundle of source-facing rays and
                               keeps the obstructions it can reach (a bit
@@ -325,8 +337,8 @@ int32_t iact_adam_step(float* params, const double* grads, float* exp_avg, float
 /* ---- launch-shape autotuner (no reference counterpart: XLA chooses its own
  * launch shapes) ------------------------------------------------------------
  * Times candidate iact_launch settings -- image layout, block size, blocks
- * per CU, source tile / sample group -- for one IMAGE or RESPONSE render of
- * the given inputs (`reps` timed renders each, after a warm-up) and writes
+ * per CU, source tile / sample group, and the automatic launch where it takes
+ * a kernel of its own -- for one IMAGE or RESPONSE render of the given inputs (`reps` timed renders each, after a warm-up) and writes
  * the fastest to *best (and its time to *best_ms, nullable).  `base` supplies
  * the fields that are kept (deterministic, accumulate; nullable).  Candidates
  * needing more workspace than given are skipped.  Synchronises `stream`;

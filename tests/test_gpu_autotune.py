@@ -41,3 +41,21 @@ def test_autotune_response_mode():
     rm0 = ia.render_response_matrix(tel, wl.sources, wl.values, "parallel")
     assert cfg.layout != 2
     np.testing.assert_allclose(rm.cpu().numpy(), rm0.cpu().numpy(), rtol=1e-5, atol=1e-7)
+
+
+def test_autotune_offers_the_automatic_launch_where_it_has_its_own_kernel():
+    """875 x 512 samples x 2048 sources behind masts: runs of samples summed at once
+    take less than half the time of any launch that traces every ray."""
+    wl = configs.workload("C3", n_sources=2048, n_samples=512)
+    tel = wl.telescope("cuda", key=2)
+    cfg = ia.autotune(tel, wl.sources, wl.values, "point", reps=2, cache=False, apply=False)
+    print(f"\n[autotune] {cfg}", flush=True)
+    assert cfg.layout == 0 and cfg.block_threads == 0 and cfg.sample_group == 0
+
+
+def test_autotune_response_without_settings_to_choose():
+    wl = configs.workload("C3", n_sources=20, n_samples=64)
+    tel = wl.telescope("cuda", key=3)
+    cfg = ia.autotune(tel, wl.sources, wl.values, "point", mode="response", cache=False,
+                      apply=False, reps=1)
+    assert vars(cfg) == vars(ia.LaunchConfig())

@@ -13,7 +13,7 @@ import torch
 import iactrace_amd as ia
 from iactrace_amd import _lib
 from iactrace_amd.render import LaunchConfig, RenderPlan
-from tests.test_gpu_tree import _sensor, _sources, _telescope
+from tests.test_gpu_tree import _sources, _telescope
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -33,7 +33,7 @@ def _all(tel, src, val, st, cot, layout=0):
 
 
 def _scene(light):
-    tel = _telescope(100, _sensor("hex"), "all", 0.0, 5, n_facets=7)
+    tel = _telescope(100, "hex", "all", 0.0, 5, n_facets=7)
     src, val, st = _sources(300, light, 3)
     cot = torch.linspace(0.5, 1.5, tel.sensors[0].n_pixels, device=DEV)
     return tel, torch.as_tensor(src, device=DEV), torch.as_tensor(val, device=DEV), st, cot
@@ -85,7 +85,7 @@ def test_tree_ends_where_its_grids_would_wrap():
     """2^24 runs of 1024 samples: the nodes' kernel would need 2^32 threads.  The
     workspace tells the kernels apart (nothing is launched): 144 bytes for each of a
     facet's three nodes beside its record, or the culling tables alone."""
-    plan = RenderPlan(_telescope(1, _sensor("square"), "all", 0.0, 5, n_facets=7))
+    plan = RenderPlan(_telescope(1, "square", "all", 0.0, 5, n_facets=7))
     sc = plan.scene([])
     L = LaunchConfig().abi()
 

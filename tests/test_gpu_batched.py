@@ -256,3 +256,29 @@ def test_c5_full_size_instances_and_fit():
     fit.close()
     print(f"[C5 fit] losses {losses}", flush=True)
     assert losses[-1] < losses[0]
+
+
+def test_fit_graph_gradients_on_the_tree_of_the_image():
+    """Instances below and above the spot tree's 128 sources: the graph's images and
+    gradients, whose walk takes over what the image's has prepared, against the
+    batched entry points on the rotations before each replay (the order of the sums
+    alone differs: 1e-6 of the largest pixel; gradients 1e-5, see test_gpu_tree)."""
+    tel, rot, s, v, off = _small_c3(5, (70, 130, 600, 0, 128))
+    bp = BatchedPlan(tel, s, v, off)
+    base = tel.mirror_groups[0].rotations.detach()
+    targets = bp.forward(base.unsqueeze(0).repeat(5, 1, 1).contiguous())
+    fit = AlignmentFit(tel, rot, s, v, off, targets, lr=1e-3)
+    for k in range(3):
+        before = fit.rotations.clone()
+        fit.step()
+        torch.cuda.synchronize()
+        want = bp.forward(before)
+        grad = bp.backward(before, fit.grad_images)
+        ei = float((fit.images - want).abs().max() / want.max())
+        eg = [float((a - b).abs().max() / b.abs().max().clamp_min(1e-30))
+              for a, b in zip(fit.grad_rotations, grad)]
+        print(f"[fit tree] replay {k}: images {ei:.1e}, gradients {max(eg):.1e}", flush=True)
+        assert ei <= 1e-6
+        assert max(eg) <= 1e-5 and float(grad.abs().max()) > 0
+        assert float((fit.rotations - before).abs().max()) > 0
+    fit.close()

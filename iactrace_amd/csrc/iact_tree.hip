@@ -1056,11 +1056,15 @@ __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B
     const int n0 = __builtin_amdgcn_readfirstlane(cnt[0]);
     const int nn = __builtin_amdgcn_readfirstlane(cnt[1]);
     // ---- patches (and, where there are few patches for the waves, segments of
-    // the list), taken by the waves one by one
+    // the list), taken by the waves one by one.  A part of one patch has as many
+    // segments as waves where four of them would be longer than a batch of 64
+    // sources (rough mirrors and near sources leave most of the list: 875 x 512
+    // samples x 300 sources behind masts, 24 arcsec: 648 us with four, 492 so)
     const int p0 = (npt * part) / (int)K.n_part, p1 = (npt * (part + 1)) / (int)K.n_part;
     const int np1 = p1 - p0;
-    const int lseg = np1 >= kWaves ? 0 : (2 * np1 >= kWaves ? 1 : 2);
-    const int nseg = 1 << lseg, nun = n0 + nn == 0 ? 0 : (p1 - p0) << lseg;
+    const int left = n0 + nn;
+    const int lseg = np1 >= kWaves ? 0 : 2 * np1 >= kWaves ? 1 : np1 > 1 || left <= 256 ? 2 : 3;
+    const int nseg = 1 << lseg, nun = left == 0 ? 0 : (p1 - p0) << lseg;
     auto take = [&]() {
       int u = 0;
       if (lane == 0) u = atomicAdd(cnt + 3, 1);

@@ -53,7 +53,7 @@ static_assert(sizeof(InstDesc) == 32 && offsetof(InstDesc, sbase) == 24,
 // A node is a run of consecutive sample records of one facet: 1024 (top), 64
 // (patch) or 16 (leaf); a facet's nodes are stored tops, patches, leaves.
 #define IACT_NODE_WORDS 32
-constexpr int kTopSamples = 1024, kPatchSamples = 64, kLeafSamples = 16;
+constexpr int kTopSamples = 1024;
 constexpr int kTreeSources = 512;  // sources of a work item, and threads of a block
 struct TreeParams {
   const float* nodes;    // (nf * per_facet, IACT_NODE_WORDS)

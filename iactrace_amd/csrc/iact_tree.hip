@@ -759,13 +759,15 @@ IACT_DEV float per_metre(float v, float ie) {                                   
 // per instruction, whatever the fraction that splits.  MODE 0: image; 1:
 // rotation gradients; 2: also positions, values, sources.
 // VALU issue bounds it (82-87 % of the busy cycles), about half in the rays of
-// unresolved leaves.  One ray per (sample, source) took 3693 us for 875 facets
-// x 1024 samples x 4096 sources without obstructions, this 960; 12732 against
-// 4200 us with 122 obstructions and a hexagonal camera, rough mirrors.  Eight
-// waves share one image, so 24 waves and their sources fit a CU; four-wave
-// blocks: 5007 against 4611 us.  Six waves per SIMD for the obstructed
-// gradients: 6.23 against 6.43 ms for the iteration above kWaves' rule; the
-// image kernels need no bound (4528 against 4537 us with one).
+// unresolved leaves.  One ray per (sample, source) took 3693 us for 382 facets
+// x 4096 samples x 4096 sources without obstructions and a square camera, this
+// 960; 12732 against 4200 us for 875 x 1024 x 16384 behind a box and four masts,
+// a hexagonal camera and smooth mirrors.  Eight waves share one image; a CU holds
+// three blocks of a kernel of up to 80 VGPRs, two of the others (obstructed
+// images 97-105, clear gradients 79-102).  Four-wave blocks: 5007 against 4611 us.
+// Six waves per SIMD for the obstructed gradients: 6.23 against 6.43 ms for an
+// iteration of five pointings; the image kernels need no bound (4528 against
+// 4537 us with one).
 template <int SRC, int KIND, int OBST, int MODE>
 __global__ __launch_bounds__(64 * kWaves)
 __attribute__((amdgpu_waves_per_eu(OBST && MODE ? 6 : 1))) void k_tree(AdjArgs B, TreeParams K) {
@@ -1555,7 +1557,8 @@ TreeLayout tree_layout(const iact_scene& sc, int ns, bool sort, int grid) {
   return T;
 }
 
-// Blocks of a full grid (24 waves per CU).
+// Blocks of a full grid (24 waves per CU: more than registers admit of some
+// kernels, whose last blocks then find the queue empty).
 int tree_max_grid(const DevInfo& dev) { return dev.n_cu * (24 / kWaves); }
 
 bool tree_serves(const TraceArgs& A, int mode, int n_acc, const DevInfo& dev, LaunchShape& shp) {
@@ -1591,7 +1594,7 @@ bool tree_serves(const TraceArgs& A, int mode, int n_acc, const DevInfo& dev, La
   const double size = sqrt((double)u.x * u.x + (double)u.y * u.y + (double)u.z * u.z) *
                       sqrt((double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z);
   if (!(fabs(det) > 1e-2 * size) || !isfinite(size) || !(size > 0.0)) return false;
-  // as many blocks as the CUs hold (160 KB of LDS each)
+  // as many blocks as the CUs' LDS holds (160 KB each)
   const int held = (int)fmin(24.0 / kWaves, floor(163840.0 / (double)lds));
   long long grid = (long long)dev.n_cu * held;
   shp.threads = 64 * kWaves;

@@ -111,14 +111,18 @@ def _surface_index(groups, device):
     return idx.to(device)
 
 
-def facets_abi(groups, keep, rotations=None, positions=None, surface_index=None):
+def facets_abi(groups, keep, rotations=None, positions=None, surface_index=None,
+               facet_counts=None):
     """IactFacets over the concatenation of stage-0 ``groups`` (render.py:201-205).
     surface_index: _surface_index of the groups where the caller holds it (made
     here, it is a copy from host memory, which waits for the stream: 16 us of a
-    60 us call on one star, and no call could be prepared while one ran)."""
+    60 us call on one star, and no call could be prepared while one ran), for
+    groups of facet_counts facets: not taken once a group's tensors were replaced
+    by others."""
     dev = groups[0].positions.device
     F = _lib.IactFacets()
-    F.n_facets = sum(len(g) for g in groups)
+    counts = [len(g) for g in groups]
+    F.n_facets = sum(counts)
     F.n_samples = groups[0].n_samples
     for g in groups:
         if g.n_samples != F.n_samples:
@@ -138,7 +142,8 @@ def facets_abi(groups, keep, rotations=None, positions=None, surface_index=None)
     # the far-source test of the kernels bounds every sample's offset from
     # its facet position by this radius
     F.max_sample_radius = max(sample_radius(g.points) for g in groups)
-    arrs["surface_index"] = _surface_index(groups, dev) if surface_index is None else surface_index
+    arrs["surface_index"] = surface_index if counts == facet_counts else \
+        _surface_index(groups, dev)
     for k, v in arrs.items():
         keep.append(v)
         setattr(F, k, v.data_ptr())
@@ -253,11 +258,8 @@ class RenderPlan:
     def scene(self, keep, rotations=None, positions=None):
         sc = _lib.IactScene.from_buffer_copy(self.static_scene)
         if self.primary:
-            counts = [len(g) for g in self.primary]
-            if counts != self.facet_counts:  # (a group's tensors were replaced by others)
-                self.surface_index = _surface_index(self.primary, self.device)
-                self.facet_counts = counts
-            sc.facets = facets_abi(self.primary, keep, rotations, positions, self.surface_index)
+            sc.facets = facets_abi(self.primary, keep, rotations, positions, self.surface_index,
+                                   self.facet_counts)
         for i, g in enumerate(self.surface_groups):
             sc.surfaces[i] = g.surface_abi()
         return sc

@@ -137,3 +137,36 @@ def test_layout_two_traces_every_ray(m, ns, sensor, obst, light):
     s, v, st = _on_device(ns, light, 4)
     _check_image(tel, s, v, st, launch=ia.LaunchConfig(layout=2, sample_group=5))
     _check_gradients(tel, s, v, st, 2)
+
+
+@pytest.mark.parametrize("wants", [("rotations",), ("rotations", "values"), ("positions",),
+                                   ("sources",)])
+@pytest.mark.parametrize("light", ["far", "near", "parallel"])
+def test_gradients_whose_tables_fit_walk_the_tree_without_its_image(wants, light):
+    """A camera whose fp64 image is too large for the tree, its fp32 gradient is not;
+    with the sums that source gradients need it is again."""
+    tel = _telescope(130, "hex", "all", 0.0, 9, n_facets=7)
+    tel = ia.Telescope(tel.mirror_groups, tel.obstruction_groups, [_large_camera("hex")])
+    ns = 140
+    assert not _takes_tree(tel, ns)
+    plan = RenderPlan(tel)
+    sc = plan.scene([])
+    own, rays = [_lib.lib().iact_bwd_workspace_size(
+        ctypes.byref(sc), ns, ctypes.byref(ia.LaunchConfig(layout=k).abi())) for k in (0, 2)]
+    assert own > rays
+    s, v, st = _on_device(ns, light, 6)
+    gen = torch.Generator().manual_seed(3)
+    cot = (0.5 + torch.rand(tel.sensors[0].n_pixels, generator=gen)).to(DEV)
+
+    def grads(layout):
+        g = tel.mirror_groups[0]
+        leaf = {"rotations": g.rotations, "positions": g.positions, "sources": s, "values": v}
+        leaf = {k: t.detach().clone().requires_grad_(k in wants) for k, t in leaf.items()}
+        t = ia.Telescope([g.replace(rotations=leaf["rotations"], positions=leaf["positions"])],
+                         tel.obstruction_groups, tel.sensors)
+        img = ia.render(t, leaf["sources"], leaf["values"], st,
+                        launch=ia.LaunchConfig(layout=layout)).reshape(-1)
+        return torch.autograd.grad(img, [leaf[k] for k in wants], cot, allow_unused=True)
+
+    for k, a, b in zip(wants, grads(1), grads(0)):
+        assert float((a.double() - b.double()).abs().max()) <= 1e-5 * float(a.abs().max()), k
